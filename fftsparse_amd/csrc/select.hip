@@ -3,32 +3,150 @@
 // row, :588-612 stripe/diffuse dynamic mask, :256-294 qk top-k, :623-641
 // columns; attn_src/fix_mask_attn/my_attn.py:39-79 for the fixed mask).
 //
-// One launch serves every head.  One workgroup (4 waves) owns RPW consecutive
-// query-block rows of one head and decides from diag_var whether the head is
-// a stripe or a diffuse head.  N <= 8192.  Stripe / fixed rows (Nk <= 4096)
-// are built word-parallel: a lane forms the 64-bit membership mask of 64 key
-// blocks (range masks for the prior, columns and causal limit; a
-// funnel-shifted window of the bit-reversed lag mask for the lag diagonals)
-// and stores it as word w of the row.  A diffuse head computes its score
-// panel S[rows][0..last row] into LDS (fp32 dot products, fixed order) in
-// passes of a few rows, so the LDS the launch reserves for the panel stays
-// small enough for four workgroups per CU.  Each wave then walks one row at a
-// time: for a diffuse row it finds the k_i-th largest score by a 32-step
-// bisection on the ordered float key with wave-wide counts, and in a single
-// ascending pass over the key blocks it evaluates the membership rule 64
-// blocks at a time, the ballot of each pass being the row's next word.
+// One launch serves every head.  Each workgroup (8 waves) decides from diag_var
+// which heads are stripe and which diffuse, and takes its share of their rows.
+// N <= 8192.
+//
+// Stripe / fixed rows (Nk <= 4096) are built word-parallel: a lane forms the
+// 64-bit membership mask of 64 key blocks (range masks for the prior, columns
+// and causal limit; a funnel-shifted window of the bit-reversed lag mask for
+// the lag diagonals) and stores it as word w of the row.
+//
+// A diffuse head's rows are taken panel_rows at a time (16 at N <= 1024): the
+// workgroup forms
+// the scores S[rows][0 .. last row] with MFMA tiles of 16 keys x 16 query rows
+// (v_mfma_f32_16x16x32 for 16-bit inputs, v_mfma_f32_16x16x4 for fp32, so
+// products and sums are fp32 as in a scalar dot product), stores them in LDS
+// as order-preserving keys, and each wave then finds the k_i-th largest key
+// of a row by bisection: ballot counts over the row's keys, held in registers
+// at N <= 1024, ending as soon as a candidate splits off exactly k_i keys
+// (about 20 of the 32 steps; only a tie at the threshold takes all 32).
+// What bounds it: the bisection's compares (16 per step and row at N = 1024)
+// and the latency of one load round.  64 KiB of LDS, two workgroups per CU.
+// The scalar form before it (each thread one key block, 2-byte loads of a row
+// per thread, 64 rows per workgroup in serial passes, 32 steps re-reading
+// LDS) took 481, 841 and 3498 us for 8 diffuse heads of 32 at N = 64, 256 and
+// 1024 (bf16, D = 128), and 444 us for one of 4 at N = 64 in fp32; this one 13,
+// 16, 41 and 13 us.
 #include <algorithm>
 
 #include "common.h"
 
 namespace fs {
 
-constexpr int kSelThreads = 256;
+constexpr int kSelThreads = 512;
 constexpr int kSelWaves = kSelThreads / 64;
 constexpr int kMaxWords = 64;                       // word-parallel path: Nk <= 4096
-constexpr int kSelMaxN = 8192;                      // per-row path: flag bytes + a one-row score panel fit the LDS budget
-constexpr int kMaxPanelRows = 16;                   // rows of a diffuse head's score panel per pass
-constexpr size_t kSelLdsBudget = 52 * 1024;         // flag bytes + score panel + q rows (three workgroups per CU)
+constexpr int kSelMaxN = 8192;
+constexpr int kHeadGroup = 64;                      // heads per row of the grid: their decisions fit one lane mask
+constexpr int kMaxGrid = 512;                       // workgroups per head group: two (64 KiB each) on each of 256 CUs
+constexpr int kPanelRows = 16;                      // an MFMA tile's query rows: the most a panel holds
+constexpr int kPanelWords = 16 * 1024;              // keys of a panel: 64 KiB, the default LDS limit of a launch
+constexpr int kRegWords = 16;                       // 64-key words of a row held in registers (N <= 1024)
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+
+// acc += A B^T of a 16-byte chunk per lane: lane l holds row l & 15 of both
+// operands, chunk l >> 4 of the step's four
+template <typename T> struct PanelMma;
+template <> struct PanelMma<bf16_t> {
+  static __device__ __forceinline__ f32x4_t go(uint4 a, uint4 b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
+                                                   0, 0, 0);
+  }
+};
+template <> struct PanelMma<f16_t> {
+  static __device__ __forceinline__ f32x4_t go(uint4 a, uint4 b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0,
+                                                  0, 0);
+  }
+};
+template <> struct PanelMma<float> {
+  // element e of every lane's chunk is one K = 4 step (the dims are added in another order)
+  static __device__ __forceinline__ f32x4_t go(uint4 a, uint4 b, f32x4_t c) {
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.x), __uint_as_float(b.x), c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.y), __uint_as_float(b.y), c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.z), __uint_as_float(b.z), c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.w), __uint_as_float(b.w), c, 0, 0, 0);
+  }
+};
+
+// elements d .. d + 16 / sizeof(T) - 1 of a row of D (0 past D, or when !ok); the
+// row itself is readable either way.  WIDE: rows are 16-byte aligned and D a
+// multiple of the chunk; the load is unconditional (clamped), so that the
+// loads of several chunks are in flight together.
+template <typename T, bool WIDE>
+__device__ __forceinline__ uint4 row_chunk(const T* row, int d, int D, bool ok) {
+  constexpr int V = 16 / sizeof(T);
+  if constexpr (WIDE) {
+    uint4 v = *reinterpret_cast<const uint4*>(row + (d < D ? d : 0));
+    const uint32_t keep = ok && d < D ? ~0u : 0u;
+    return make_uint4(v.x & keep, v.y & keep, v.z & keep, v.w & keep);
+  } else {
+    T e[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const T v = row[d + i < D ? d + i : 0];
+      e[i] = ok && d + i < D ? v : T{0};
+    }
+    return __builtin_bit_cast(uint4, e);
+  }
+}
+
+// Score panel of a diffuse head's rows r0 .. r0 + nrows - 1 (nrows <= 16) against keys 0 .. r0 + nrows - 1:
+// S[i][j] = (q_b[i] . k_b[j]) * (1/sqrt(D)) (:234-249), as order-preserving keys.  Key j of row rr is word
+// (chunk j / 4, swizzled by the row) of the row's `stride` words: the 16 rows' chunk stores of one tile fall
+// on different banks, a row's 64 consecutive keys on 64 different ones.
+template <typename T, bool WIDE>
+__device__ __forceinline__ void score_panel(const T* qb, const T* kb, int D, int r0, int nrows, float inv_sqrt_d,
+                                            uint32_t* panel, int stride, int lane) {
+  constexpr int V = 16 / (int)sizeof(T);
+  constexpr int kSteps = 128 / (4 * V);            // MFMA steps per 128 dims (dims past D are zero)
+  constexpr int kTiles = !WIDE ? 1 : (sizeof(T) == 2 ? 4 : 2);   // key tiles in flight per wave
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const int jmax = r0 + nrows, ntile = (jmax + 15) >> 4;
+  const bool qok = l16 < nrows;
+  const T* qrow = qb + (int64_t)(r0 + (qok ? l16 : 0)) * D;
+  for (int t0 = wave * kTiles; t0 < ntile; t0 += kSelWaves * kTiles) {
+    f32x4_t acc[kTiles];
+#pragma unroll
+    for (int u = 0; u < kTiles; ++u) acc[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int d0 = 0; d0 < D; d0 += 128) {
+      uint4 qv[kSteps], kv[kTiles][kSteps];
+#pragma unroll
+      for (int st = 0; st < kSteps; ++st) qv[st] = row_chunk<T, WIDE>(qrow, d0 + (4 * st + g) * V, D, qok);
+#pragma unroll
+      for (int u = 0; u < kTiles; ++u) {
+        const int j = (t0 + u) * 16 + l16;
+        const T* krow = kb + (int64_t)min(j, jmax - 1) * D;   // keys past the last row: read, never counted
+#pragma unroll
+        for (int st = 0; st < kSteps; ++st) kv[u][st] = row_chunk<T, WIDE>(krow, d0 + (4 * st + g) * V, D, true);
+      }
+#pragma unroll
+      for (int st = 0; st < kSteps; ++st)
+#pragma unroll
+        for (int u = 0; u < kTiles; ++u) acc[u] = PanelMma<T>::go(kv[u][st], qv[st], acc[u]);
+    }
+    // a fixed wait between the chain and the first read of its results, whatever path leads here
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 15" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    // lane: keys 16 t + 4 g .. + 3 of query row l16
+#pragma unroll
+    for (int u = 0; u < kTiles; ++u) {
+      const int c = (t0 + u) * 4 + g;              // 4-key chunk of the row
+      if (t0 + u < ntile && qok) {
+        uint32_t w[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) w[r] = order_key(acc[u][r] * inv_sqrt_d);
+        *reinterpret_cast<uint4*>(panel + l16 * stride + (c ^ l16) * 4) = make_uint4(w[0], w[1], w[2], w[3]);
+      }
+    }
+  }
+}
 
 // LDS of the word-parallel path (the start of the launch's dynamic LDS)
 struct WordRowsLds {
@@ -45,31 +163,21 @@ __device__ __forceinline__ uint64_t range_bits(int w, int lo, int hi) {
   return upto & ~((1ull << b0) - 1);
 }
 
-// panel_rows: rows of a diffuse head's score panel per pass (0 without the
-// dynamic mask).  Dynamic LDS: WordRowsLds (word-parallel rows) or, for the
-// per-row path, the head's flag bytes [N], then the panel [panel_rows][N] and
-// the pass's q rows [panel_rows][D].
-template <typename T>
-__global__ __launch_bounds__(kSelThreads) void select_kernel(fs_select_args a, int rows_per_wave, int panel_rows,
-                                                             float inv_sqrt_d) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char sel_lds[];
-  const int RPW = rows_per_wave * kSelWaves;
-  const int N = a.N, Nk = a.Nk, D = a.D;
-  const int chunks = (N + RPW - 1) / RPW;
-  const int h = blockIdx.x / chunks;
-  const int r0 = (blockIdx.x - h * chunks) * RPW;
-  const int hk = h / (a.Hq / a.Hk);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int NW = (Nk + 63) >> 6;                   // 64-block words per row
-  const bool word_rows = NW <= kMaxWords;          // stripe / fixed rows are built word-parallel (below)
-
-  // The word-parallel path stages the head's lag / column / last-row flags.
-  // Their loads are issued here, before the decision's, so that one wait
-  // covers both: flag bytes j = 4 w .. 4 w + 3 of word w = tid + 256 u.
+// Rows r0 .. r0 + RPW - 1 of a stripe head or of a fixed mask (every thread of the workgroup).
+__device__ void stripe_rows_of(const fs_select_args& a, int h, int r0, int RPW, unsigned char* sel_lds) {
+  const int N = a.N, Nk = a.Nk;
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));                    // keeps the lane's addresses out of the item loop's preheader
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int NW = (Nk + 63) >> 6;
+  const bool words = NW <= kMaxWords;              // built word-parallel
+  const bool use_lags = a.dyn_mode == 1, use_cols = a.col_mode != 0;
+  // The word-parallel path stages the head's lag / column / last-row flags:
+  // bytes j = 4 w .. 4 w + 3 of word w = tid + 512 u, every load before the first wait.
   constexpr int kFlagWords = 4096 / 4 / kSelThreads;
   uint32_t fkr[kFlagWords], fcr[kFlagWords], flr[kFlagWords];
   const int nw4 = (N + 3) >> 2;
-  if (word_rows) {                                 // (loaded for a diffuse head too: the decision comes later)
+  if (words) {
     const int64_t hb = (int64_t)h * N;
     const bool v4 = (N & 3) == 0;                  // row starts 4-byte aligned (buffers are)
 #pragma unroll
@@ -91,31 +199,6 @@ __global__ __launch_bounds__(kSelThreads) void select_kernel(fs_select_args a, i
       }
     }
   }
-
-  // ---- stripe / diffuse decision (:359-363); identical in every workgroup of the head
-  bool stripe = false;
-  if (a.dyn_mode == 1) {
-    float mv;
-    if (a.stripe_all_diffuse) {
-      mv = INFINITY;
-    } else {
-      // every wave forms the same sum (butterfly order is lane-independent)
-      float s = 0.f;
-      for (int i = lane; i < a.n_samples; i += 64) s += a.diag_var[(int64_t)h * a.n_samples + i];
-      s = wave_sum(s);
-      mv = s / (float)a.n_samples;
-      stripe = mv <= a.stripe_threshold;        // false for nan
-    }
-    if (r0 == 0 && tid == 0) {
-      if (a.mean_var) a.mean_var[h] = mv;
-      if (a.is_stripe) a.is_stripe[h] = stripe ? 1 : 0;
-    }
-  }
-  const bool diffuse = a.dyn_mode == 1 && !stripe;
-  const bool words = word_rows && !diffuse;
-  const bool use_lags = a.dyn_mode == 1 && stripe;
-  const bool use_cols = a.col_mode == 2 || (a.col_mode == 1 && stripe);
-  const int rend = min(N, r0 + RPW);
 
   const int lw = a.local_window;
   const bool has_last = a.last_sel != nullptr;
@@ -195,8 +278,6 @@ __global__ __launch_bounds__(kSelThreads) void select_kernel(fs_select_args a, i
   }
   // ---- per-head lag / column / last-row flags, staged in LDS (bit 0 lag, 1 column, 2 last row)
   uint8_t* flags = sel_lds;
-  float* panel = reinterpret_cast<float*>(sel_lds + ((N + 15) & ~15));   // [panel_rows][N]
-  float* qrows = panel + (size_t)panel_rows * N;                           // [panel_rows][D]
   for (int j = tid; j < N; j += kSelThreads) {
     uint8_t f = 0;
     if (a.keep_tau && a.keep_tau[(int64_t)h * N + j]) f |= 1;
@@ -205,109 +286,230 @@ __global__ __launch_bounds__(kSelThreads) void select_kernel(fs_select_args a, i
     flags[j] = f;
   }
   __syncthreads();
-
-  // rows r0 + p0 .. r0 + pend - 1 per pass: a diffuse head's panel holds
-  // panel_rows rows; other heads take all their rows in one pass
-  const int P = diffuse ? panel_rows : RPW;
   const int nrows = min(RPW, N - r0);
-  for (int p0 = 0; p0 < nrows; p0 += P) {
-    const int pend = min(nrows, p0 + P);
-    if (diffuse) {
-      // ---- score panel S[i][j] = (q_b[i] . k_b[j]) * (1/sqrt(D)), j <= last row of the pass (:234-249)
-      const T* qb = static_cast<const T*>(a.q_b) + (int64_t)h * N * D;
-      const T* kb = static_cast<const T*>(a.k_b) + (int64_t)hk * N * D;
-      __syncthreads();                             // the previous pass is done with the panel
-      for (int e = tid; e < P * D; e += kSelThreads) {
-        const int rr = e / D, d = e - rr * D;
-        qrows[e] = (p0 + rr < pend) ? to_f32(qb[(int64_t)(r0 + p0 + rr) * D + d]) : 0.f;
-      }
-      __syncthreads();
-      const int jmax = r0 + pend;                  // columns 0 .. the pass's last row
-      for (int j = tid; j < jmax; j += kSelThreads) {
-        float acc[kMaxPanelRows];
-#pragma unroll
-        for (int rr = 0; rr < kMaxPanelRows; ++rr) acc[rr] = 0.f;
-        const T* kr = kb + (int64_t)j * D;
-        for (int d = 0; d < D; ++d) {
-          const float kv = to_f32(kr[d]);
-#pragma unroll
-          for (int rr = 0; rr < kMaxPanelRows; ++rr)
-            if (rr < P) acc[rr] += qrows[rr * D + d] * kv;
+  for (int rr = wave; rr < nrows; rr += kSelWaves) {
+    const int i = r0 + rr;
+    const int jlim = a.mask_causal ? min(i + 1, Nk) : Nk;
+    // ---- membership in ascending block order, one word per 64 blocks
+    uint64_t* out = a.blk_bits + ((int64_t)h * N + i) * NW;
+    int cnt = 0;
+    for (int j0 = 0; j0 < jlim; j0 += 64) {
+      const int j = j0 + lane;
+      bool in = false;
+      if (j < jlim) {
+        // prior (:83-95): sink | recent | local window
+        in = j < a.keep_sink || j >= Nk - a.keep_recent || (lw > 0 && abs(i - j) <= lw);
+        const uint8_t fj = j < N ? flags[j] : 0;
+        if (has_last && i == N - 1 && (fj & 4)) in = true;
+        if (use_lags) {
+          const int t = i - j;
+          if (t >= a.remote_start && j >= a.keep_sink && (flags[t] & 1)) in = true;
         }
-#pragma unroll
-        for (int rr = 0; rr < kMaxPanelRows; ++rr)
-          if (rr < P) panel[(size_t)rr * N + j] = acc[rr] * inv_sqrt_d;
+        if (use_cols && j <= i && (fj & 2)) in = true;
       }
-      __syncthreads();
+      const uint64_t m = __ballot(in);
+      if (lane == 0) out[j0 >> 6] = m;
+      cnt += __popcll(m);
     }
-    for (int rr = p0 + wave; rr < pend; rr += kSelWaves) {
-      const int i = r0 + rr;
-      const int jlim = a.mask_causal ? min(i + 1, Nk) : Nk;
-      const float* srow = panel + (size_t)(rr - p0) * N;
-      // ---- diffuse row: k_i-th largest of S[i][0..i] (:271-276)
-      uint32_t thr = 0;
-      int need = 0;
-      if (diffuse) {
-        int k = (int)((float)(i + 1) * a.qk_topk_ratio);
-        if (k < 1) k = 1;
-        const int n = i + 1;
-        if (k > n) k = n;
-        uint32_t prefix = 0;
-        for (int b = 31; b >= 0; --b) {
-          const uint32_t cand = prefix | (1u << b);
-          int c = 0;
-          for (int j0 = 0; j0 < n; j0 += 64) c += wave_count(j0 + lane < n && order_key(srow[j0 + lane]) >= cand);
-          if (c >= k) prefix = cand;
+    for (int w = ((jlim + 63) >> 6) + lane; w < NW; w += 64) out[w] = 0ull;   // words past the causal limit
+    if (lane == 0) a.blk_cnt[(int64_t)h * N + i] = cnt;
+  }
+}
+
+// Rows r0 .. r0 + panel_rows - 1 of a diffuse head (every thread of the workgroup).
+template <typename T>
+__device__ void diffuse_rows(const fs_select_args& a, int h, int r0, int panel_rows, float inv_sqrt_d,
+                             uint32_t* panel) {
+  const int N = a.N, Nk = a.Nk, D = a.D, hk = h / (a.Hq / a.Hk);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));                   // keeps the lane's addresses out of the item loop's preheader
+  const int NW = (Nk + 63) >> 6;
+  const int lw = a.local_window;
+  const bool has_last = a.last_sel != nullptr, use_cols = a.col_mode == 2;
+  const int stride = (N + 63) & ~63;
+  const int nrows = min(panel_rows, N - r0);
+  const T* qb = static_cast<const T*>(a.q_b) + (int64_t)h * N * D;
+  const T* kb = static_cast<const T*>(a.k_b) + (int64_t)hk * N * D;
+  if (D % (16 / (int)sizeof(T)) == 0 && (((uintptr_t)a.q_b | (uintptr_t)a.k_b) & 15) == 0)
+    score_panel<T, true>(qb, kb, D, r0, nrows, inv_sqrt_d, panel, stride, lane);
+  else
+    score_panel<T, false>(qb, kb, D, r0, nrows, inv_sqrt_d, panel, stride, lane);
+  __syncthreads();
+  for (int rr = wave; rr < nrows; rr += kSelWaves) {
+    const int i = r0 + rr, n = i + 1, nw = (n + 63) >> 6;
+    const uint32_t* srow = panel + rr * stride;
+    auto key_at = [&](int j) -> uint32_t { return srow[((j >> 2) ^ rr) * 4 + (j & 3)]; };   // j < n rounded up to 64
+    // ---- the k_i-th largest of S[i][0..i] (:271-276).  Keys past the row are 0, below every candidate.
+    int k = (int)((float)n * a.qk_topk_ratio);
+    k = min(max(k, 1), n);
+    uint32_t x[kRegWords];
+    const bool held = nw <= kRegWords;
+    if (held) {
+#pragma unroll
+      for (int u = 0; u < kRegWords; ++u) x[u] = 64 * u + lane < n ? key_at(64 * u + lane) : 0u;
+    }
+    // keys >= cand (cand > 0), over whole groups of four words
+    auto count_ge = [&](uint32_t cand) -> int {
+      int c = 0;
+      if (held) {
+#pragma unroll
+        for (int q = 0; q < kRegWords / 4; ++q) {
+          if (4 * q >= nw) break;
+#pragma unroll
+          for (int u = 4 * q; u < 4 * q + 4; ++u) c += wave_count(x[u] >= cand);
         }
-        int gt = 0;
-        for (int j0 = 0; j0 < n; j0 += 64) gt += wave_count(j0 + lane < n && order_key(srow[j0 + lane]) > prefix);
-        thr = prefix;
-        need = k - gt;
+      } else {
+        const int full = n >> 6;                   // words with every key in the row
+        int u0 = 0;
+        for (; u0 + 8 <= full; u0 += 8) {          // eight reads in flight
+          uint32_t y[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) y[u] = key_at(64 * (u0 + u) + lane);
+#pragma unroll
+          for (int u = 0; u < 8; ++u) c += wave_count(y[u] >= cand);
+        }
+        for (; u0 < full; ++u0) c += wave_count(key_at(64 * u0 + lane) >= cand);
+        if (full < nw) c += wave_count(64 * full + lane < n && key_at(64 * full + lane) >= cand);
       }
-      // ---- membership in ascending block order, one word per 64 blocks
-      uint64_t* out = a.blk_bits + ((int64_t)h * N + i) * NW;
-      int cnt = 0, eq_seen = 0;
-      for (int j0 = 0; j0 < jlim; j0 += 64) {
-        const int j = j0 + lane;
-        const bool valid = j < jlim;
-        bool in = false;
-        bool eq = false;
-        if (valid) {
-          // prior (:83-95): sink | recent | local window
-          in = j < a.keep_sink || j >= Nk - a.keep_recent || (lw > 0 && abs(i - j) <= lw);
-          const uint8_t fj = j < N ? flags[j] : 0;
-          if (has_last && i == N - 1 && (fj & 4)) in = true;
-          if (use_lags) {
-            const int t = i - j;
-            if (t >= a.remote_start && j >= a.keep_sink && (flags[t] & 1)) in = true;
-          }
-          if (diffuse && j <= i) {
-            const uint32_t key = order_key(srow[j]);
-            if (key > thr) in = true;
-            eq = key == thr;
-          }
-          if (use_cols && j <= i && (fj & 2)) in = true;
+      return c;
+    };
+    // thr: every larger key is selected, and the first `need` keys equal to it
+    uint32_t thr = 0;
+    int need = 0;
+    bool split = false;                            // a candidate split off exactly k keys: no ties to rank
+    for (int b = 31; b >= 0 && !split; --b) {
+      const uint32_t cand = thr | (1u << b);
+      const int c = count_ge(cand);
+      if (c >= k) thr = cand;
+      split = c == k;
+    }
+    if (split) thr -= 1;
+    else need = k - (thr == 0xffffffffu ? 0 : count_ge(thr + 1));
+    // ---- the row's words, word w0 + l kept by lane l: the top-k ballots, then (word-parallel) the prior
+    // (:83-95), the last row's and the columns' words
+    const int jlim = a.mask_causal ? min(n, Nk) : Nk;
+    uint64_t* out = a.blk_bits + ((int64_t)h * N + i) * NW;
+    const bool extra = use_cols || (has_last && i == N - 1);
+    int cnt = 0, eq_seen = 0;
+    for (int w0 = 0; w0 < NW; w0 += 64) {
+      uint32_t mlo = 0, mhi = 0;
+      auto put = [&](int w, uint64_t m) {          // |= m in lane w - w0
+        if (lane == w - w0) {
+          mlo |= (uint32_t)m;
+          mhi |= (uint32_t)(m >> 32);
         }
-        if (diffuse) {
+      };
+      for (int w = w0; w < min(nw, w0 + 64); ++w) {
+        const int j = 64 * w + lane;
+        const uint32_t key = j < n ? key_at(j) : 0u;
+        bool in = key > thr;
+        if (need > 0) {
+          const bool eq = j < n && key == thr;
           const uint64_t me = __ballot(eq);
-          if (eq && eq_seen + rank_below(me) < need) in = true;
+          in = in || (eq && eq_seen + rank_below(me) < need);
           eq_seen += __popcll(me);
         }
-        const uint64_t m = __ballot(in);
-        if (lane == 0) out[j0 >> 6] = m;
+        put(w, __ballot(in));
+      }
+      if (extra) {
+        for (int w = w0; w < min(NW, w0 + 64); ++w) {
+          const int j = 64 * w + lane;
+          bool in = has_last && i == N - 1 && j < N && a.last_sel[(int64_t)h * N + j] != 0;
+          if (use_cols && j < n) in = in || a.col_sel[(int64_t)h * N + j] != 0;
+          put(w, __ballot(in));
+        }
+      }
+      const int w = w0 + lane;
+      uint64_t m = (uint64_t)mhi << 32 | mlo;
+      m |= range_bits(w, 0, a.keep_sink) | range_bits(w, Nk - a.keep_recent, Nk);
+      if (lw > 0) m |= range_bits(w, i - lw, i + lw + 1);
+      m &= range_bits(w, 0, jlim);
+      if (w < NW) {
+        out[w] = m;
         cnt += __popcll(m);
       }
-      for (int w = ((jlim + 63) >> 6) + lane; w < NW; w += 64) out[w] = 0ull;   // words past the causal limit
-      if (lane == 0) a.blk_cnt[(int64_t)h * N + i] = cnt;
+    }
+    cnt = wave_sum_i(cnt);
+    if (lane == 0) a.blk_cnt[(int64_t)h * N + i] = cnt;
+  }
+}
+
+// The head group's work, dealt to the launch's workgroups.  blockIdx.y: heads
+// 64 blockIdx.y ..; every workgroup decides its group's heads (each wave some of
+// them), so the items -- panel_rows rows of a diffuse head, the latest rows (the
+// longest) first, then stripe_rows rows of a stripe or fixed head -- are
+// enumerated without a list in memory, and workgroup b takes items b, b +
+// gridDim.x, ..  (One workgroup per panel_rows rows of every head instead, the
+// stripe heads' spare ones returning: 21.6 against 10.1 us on 32 stripe heads of
+// 1024 blocks, the 64 KiB workgroups going through four rounds.)
+// Dynamic LDS: WordRowsLds (word-parallel rows), the head's flag bytes [N]
+// (other stripe rows), or the panel [panel_rows][N rounded up to 64] of keys.
+template <typename T>
+__global__ __launch_bounds__(kSelThreads) __attribute__((amdgpu_waves_per_eu(4))) void select_kernel(
+    fs_select_args a, int stripe_rows, int panel_rows, float inv_sqrt_d) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char sel_lds[];
+  __shared__ uint8_t is_diffuse[kHeadGroup];
+  const int N = a.N, Nk = a.Nk, D = a.D;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: what follows from it branches on scalars
+  const int NW = (Nk + 63) >> 6;                   // 64-block words per row
+  const int h0 = blockIdx.y * kHeadGroup, nh = min(kHeadGroup, a.Hq - h0);
+
+  // ---- stripe / diffuse decisions (:359-363): wave w takes heads w, w + 8, .., four at a time
+  uint64_t dmask = 0;                              // bit e: head h0 + e is diffuse
+  if (a.dyn_mode == 1) {
+    for (int e0 = wave; e0 < nh; e0 += 4 * kSelWaves) {
+      float s[4] = {0.f, 0.f, 0.f, 0.f};
+      if (!a.stripe_all_diffuse) {
+        for (int i = lane; i < a.n_samples; i += 64) {
+          float d[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            d[u] = a.diag_var[(int64_t)(h0 + min(e0 + u * kSelWaves, nh - 1)) * a.n_samples + i];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) s[u] += d[u];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int e = e0 + u * kSelWaves;
+        s[u] = wave_sum(s[u]);
+        const float mv = a.stripe_all_diffuse ? INFINITY : s[u] / (float)a.n_samples;
+        const bool stripe = mv <= a.stripe_threshold && !a.stripe_all_diffuse;   // false for nan
+        if (lane == 0 && e < nh) {
+          is_diffuse[e] = stripe ? 0 : 1;
+          if (blockIdx.x == 0) {
+            if (a.mean_var) a.mean_var[h0 + e] = mv;
+            if (a.is_stripe) a.is_stripe[h0 + e] = stripe ? 1 : 0;
+          }
+        }
+      }
+    }
+    __syncthreads();
+    dmask = __ballot(lane < nh && is_diffuse[lane] != 0);
+  }
+  const uint64_t hmask = nh == 64 ? ~0ull : (1ull << nh) - 1;
+  const int nd = __popcll(dmask), ns = nh - nd;
+  const int dchunks = (N + panel_rows - 1) / panel_rows, schunks = (N + stripe_rows - 1) / stripe_rows;
+  const int ditems = nd * dchunks, items = ditems + ns * schunks;
+  for (int item = blockIdx.x; item < items; item += gridDim.x) {
+    if (item != (int)blockIdx.x) __syncthreads();  // the previous item's LDS is read
+    if (item < ditems) {
+      diffuse_rows<T>(a, h0 + nth_set_bit(dmask, item % nd), (dchunks - 1 - item / nd) * panel_rows, panel_rows,
+                      inv_sqrt_d, reinterpret_cast<uint32_t*>(sel_lds));
+    } else {
+      const int it = item - ditems, e = it / schunks;
+      stripe_rows_of(a, h0 + nth_set_bit(hmask & ~dmask, e), (it - e * schunks) * stripe_rows, stripe_rows, sel_lds);
     }
   }
 }
 
 template <typename T>
-static int launch_select(const fs_select_args& a, unsigned grid, size_t smem, int rows_per_wave, int panel_rows,
+static int launch_select(const fs_select_args& a, dim3 grid, size_t smem, int stripe_rows, int panel_rows,
                          float inv_sqrt_d, hipStream_t s) {
   if (int rc = fs_host::allow_dynamic_lds(select_kernel<T>, smem, "fs_select")) return rc;
-  select_kernel<T><<<grid, kSelThreads, smem, s>>>(a, rows_per_wave, panel_rows, inv_sqrt_d);
+  select_kernel<T><<<grid, kSelThreads, smem, s>>>(a, stripe_rows, panel_rows, inv_sqrt_d);
   return 0;
 }
 
@@ -332,33 +534,32 @@ extern "C" int fs_select(const fs_select_args* a, void* stream) {
                "fs_select: dynamic, column and last-row masks need N == Nk");
   FS_CHECK_SUPPORTED(a->N <= kSelMaxN && (a->dyn_mode == 0 || a->D <= 256), "fs_select: N=%d > %d or D=%d > 256",
                      a->N, kSelMaxN, a->D);
-  // rows per wave: 16 word-parallel rows of <= 1024 blocks (four rows per
-  // pass of 16 lanes each), fewer for longer rows; one on the per-row path
+  // Rows of a stripe or fixed head's work item: 64 word-parallel rows of <= 1024
+  // blocks (four rows per wave pass of 16 lanes each), fewer for longer rows; one
+  // per wave on the per-row path.  Rows of a diffuse head's: what a 64 KiB panel
+  // holds, at most one MFMA tile's 16.
   const int NW = (a->Nk + 63) / 64;
-  const int rows_per_wave = NW <= 16 ? 16 : (NW <= 32 ? 8 : (NW <= kMaxWords ? 4 : 1));
-  const int RPW = rows_per_wave * kSelWaves;
-  const int chunks = (a->N + RPW - 1) / RPW;
-  const float inv_sqrt_d = a->D > 0 ? 1.0f / (float)sqrt((double)a->D) : 1.0f;
-  // dynamic LDS: the word-parallel path's, or flag bytes + a diffuse head's
-  // panel of panel_rows rows (a multiple of 4 rows when 4 fit) + its q rows
-  const size_t flag_bytes = ((size_t)a->N + 15) & ~(size_t)15;
-  int panel_rows = 0;
+  const int stripe_rows = NW <= 16 ? 64 : (NW <= 32 ? 32 : (NW <= kMaxWords ? 16 : kSelWaves));
+  int panel_rows = stripe_rows;
+  size_t smem = ((size_t)a->N + 15) & ~(size_t)15;
   if (a->dyn_mode == 1) {
-    const size_t per_row = (size_t)(a->N + a->D) * sizeof(float);
-    panel_rows = (int)std::min<size_t>((kSelLdsBudget - flag_bytes) / per_row, (size_t)std::min(RPW, kMaxPanelRows));
-    if (panel_rows >= 4) panel_rows &= ~3;
-    panel_rows = std::max(panel_rows, 1);
+    const int stride = (a->N + 63) & ~63;
+    panel_rows = kPanelRows;
+    while (panel_rows * stride > kPanelWords) panel_rows >>= 1;   // 2 at N = 8192
+    smem = std::max(smem, (size_t)panel_rows * stride * sizeof(uint32_t));
   }
-  size_t smem = flag_bytes + (size_t)panel_rows * (a->N + a->D) * sizeof(float);
   if (NW <= kMaxWords) smem = std::max(smem, sizeof(WordRowsLds));
+  // the most items a head group can have: every head diffuse
+  const int64_t items = (int64_t)std::min(a->Hq, kHeadGroup) * ((a->N + panel_rows - 1) / panel_rows);
+  const dim3 grid((unsigned)std::min<int64_t>(items, kMaxGrid), (unsigned)((a->Hq + kHeadGroup - 1) / kHeadGroup));
+  const float inv_sqrt_d = a->D > 0 ? 1.0f / (float)sqrt((double)a->D) : 1.0f;
   hipStream_t s = (hipStream_t)stream;
-  const unsigned grid = (unsigned)(a->Hq * chunks);
   const int dt = a->dyn_mode == 1 ? a->dtype : FS_DTYPE_F32;
   int rc = 0;
   switch (dt) {
-    case FS_DTYPE_F32: rc = launch_select<float>(*a, grid, smem, rows_per_wave, panel_rows, inv_sqrt_d, s); break;
-    case FS_DTYPE_BF16: rc = launch_select<bf16_t>(*a, grid, smem, rows_per_wave, panel_rows, inv_sqrt_d, s); break;
-    case FS_DTYPE_F16: rc = launch_select<f16_t>(*a, grid, smem, rows_per_wave, panel_rows, inv_sqrt_d, s); break;
+    case FS_DTYPE_F32: rc = launch_select<float>(*a, grid, smem, stripe_rows, panel_rows, inv_sqrt_d, s); break;
+    case FS_DTYPE_BF16: rc = launch_select<bf16_t>(*a, grid, smem, stripe_rows, panel_rows, inv_sqrt_d, s); break;
+    case FS_DTYPE_F16: rc = launch_select<f16_t>(*a, grid, smem, stripe_rows, panel_rows, inv_sqrt_d, s); break;
     default: fs_host::set_error("fs_select: dtype %d unsupported", a->dtype); return FS_ERR_UNSUPPORTED;
   }
   if (rc) return rc;
