@@ -2,8 +2,8 @@
 // Role: block_sparse_attn_func (my_attn_v7.py:775-786) and, with no block
 // list, flash_attn_func(causal=True) (my_attn_v7.py:509-519).
 //
-// Pre-pass (vt_kernel): V [Lk][D] of every KV head is rewritten once per call
-// as V^T [D][Lp] (Lp = Nk * BS rounded up to 64, zero padded) with the keys of every group of
+// Pre-pass (vt_kernel; not where v_direct holds, see VD): V [Lk][D] of every KV
+// head is rewritten once per call as V^T [D][Lp] (Lp = Nk * BS rounded up to 64, zero padded) with the keys of every group of
 // 16 stored in the order 0-3, 8-11, 4-7, 12-15.  With 16- or 32-token block
 // lists (union mode) V^T is stored block by block instead, [Lp / bs][D][bs]:
 // the copy of one listed block is then one contiguous run of D * bs keys
@@ -53,6 +53,7 @@ namespace fs {
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef short i16x4_t __attribute__((ext_vector_type(4)));
 
 template <typename T> struct MfmaOps;
 template <> struct MfmaOps<bf16_t> {
@@ -102,6 +103,11 @@ template <> struct MfmaOps<f16_t> {
     return acc;
   }
 };
+
+// the 8 elements of two transposing LDS reads (V read as it is stored, see below)
+__device__ __forceinline__ uint4 join8(i16x4_t a, i16x4_t b) {
+  return __builtin_bit_cast(uint4, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+}
 
 constexpr int kD = 128;
 
@@ -187,12 +193,15 @@ __device__ __forceinline__ void dma16s(uint32_t lds_base, const void* sbase, uin
                :: "s"(lds_base), "v"(voff), "s"(sbase) : "memory");
 }
 
+// a row of zeros to copy for keys past the sequence
+static __device__ const uint4 kZeroRow[kD * 2 / 16] = {};
+
 // Arguments of the main kernel: the subset of fs_attn_args it reads, with the
 // per-row strides narrowed to 32 bits (checked on the host).
 struct AttnKArgs {
   const uint16_t* q;
   const uint16_t* k;
-  const uint16_t* vt;
+  const uint16_t* v;            // V^T of the workspace, or V itself (VD)
   uint16_t* out;
   const int32_t* blk_cnt;       // work order only (non-null: block masks given)
   const uint64_t* blk_bits;     // [Hq][Nq][NWk] block mask rows (64-token and longer blocks)
@@ -210,8 +219,20 @@ struct AttnKArgs {
   // last pool_units are taken by whichever XCD asks first
   int32_t* ctr;
   int static_units, pool_units;
+  int v_sl;                     // VD only: V's strides
+  int64_t v_sb, v_sh;
 };
 
+// 4 16-bit elements per lane of a transposing LDS read (VD, below)
+__device__ __forceinline__ i16x4_t lds_tr8(const char* base, uint32_t off) {
+  typedef __attribute__((address_space(3))) i16x4_t* lptr;
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lptr)(base + off));
+}
+// VD: 16-byte chunk c of key row r of a V tile is stored at chunk c ^ v_swz(r)
+template <int D>
+__device__ __forceinline__ int v_swz(int r) {
+  return D == 128 ? (r & 3) << 2 : ((r >> 1) & 1) << 2;
+}
 // 16-byte LDS operand at byte offset off of base
 __device__ __forceinline__ uint4 lds16(const char* base, uint32_t off) {
   return *reinterpret_cast<const uint4*>(base + off);
@@ -224,7 +245,13 @@ __device__ __forceinline__ uint4 lds16(const char* base, uint32_t off) {
 // block its row did not select are masked.  A tile of TK keys holds TK / LB
 // union entries, so every K / V^T tile copy serves 128 queries and every wave
 // does 32 x TK per barrier, as with 128-token blocks.
-template <int BS, int TK, typename T, int LB = BS, int D = kD>
+//
+// VD (V direct): no V^T pre-pass.  V tiles are copied as they are, [TK][D], and
+// each operand of P V is two transposing LDS reads (ds_read_b64_tr_b16) instead
+// of one ds_read_b128 of V^T.  The loop is 1-3% slower that way (the operand
+// reads are 1.5 times as many instructions), and the pre-pass's launch and its
+// read and write of V are saved; see v_direct for where the line lies.
+template <int BS, int TK, typename T, int LB = BS, int D = kD, bool VD = false>
 __global__ __launch_bounds__((AttnCfg<BS, TK, D>::NT)) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void bsattn_kernel(AttnKArgs a) {
   using C = AttnCfg<BS, TK, D>;
@@ -234,6 +261,7 @@ void bsattn_kernel(AttnKArgs a) {
   constexpr int ROWB = D * 2, CPR = D / 8, SWM = CPR - 1, RPR = 1024 / ROWB, LCPR = D == 128 ? 4 : 3;
   constexpr bool UNION = LB < BS;
   constexpr int EPT = UNION ? TK / LB : 1;         // union entries per tile
+  static_assert(!(UNION && VD), "union mode reads V^T");
   static_assert(!UNION || (BS == 128 && TK == 64 && (LB == 16 || LB == 32)), "union mode: 16- or 32-token lists");
   using Ops = MfmaOps<T>;
   using V8 = typename Ops::V8;
@@ -316,7 +344,7 @@ void bsattn_kernel(AttnKArgs a) {
   const int kbase = kh * C::KH;
   const uint16_t* qp = a.q + b * a.q_sb + h * a.q_sh;
   const uint16_t* kp = a.k + b * a.k_sb + hk * a.k_sh;
-  const uint16_t* vtp = a.vt + (int64_t)(b * a.Hk + hk) * D * a.Lp;
+  const uint16_t* vp = VD ? a.v + b * a.v_sb + hk * a.v_sh : a.v + (int64_t)(b * a.Hk + hk) * D * a.Lp;
   const int q0 = qb * BS;
   const int off = a.Lk - a.Lq;
   const int qw0 = q0 + qq * 32;                 // first query of this wave
@@ -431,6 +459,8 @@ void bsattn_kernel(AttnKArgs a) {
       voff[i] = (TK == 128 ? (uint32_t)(r * a.Lp + c * 8)                          // d = r
                            : (uint32_t)((2 * r + (c >> 3)) * a.Lp + (c & 7) * 8))  // two d rows per LDS row
                 * 2u;
+      // VD: key rows like K's
+      if constexpr (VD) voff[i] = (uint32_t)(rk * a.v_sl + ((lane & SWM) ^ v_swz<D>(rk)) * 8) * 2u;
     }
   }
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)&lds[0][0][0]);
@@ -506,14 +536,34 @@ void bsattn_kernel(AttnKArgs a) {
           uint32_t k = ek[0];
 #pragma unroll
           for (int ie = 1; ie < EPT; ++ie) k = sel == ie ? ek[ie] : k;
-          dma16s(lv + i * 1024, vtp, voff[i] + k);
+          dma16s(lv + i * 1024, vp, voff[i] + k);
         }
         return;
       }
     }
-    const uint16_t* base = vtp + max(key0, 0);     // V^T is zero padded to Lp
+    if constexpr (VD) {
+      if (key0 >= 0 && key0 + TK <= a.Lk) {
+        const uint16_t* base = vp + (int64_t)key0 * a.v_sl;
 #pragma unroll
-    for (int i = 0; i < NR; ++i) dma16s(lv + i * 1024, base, voff[i]);
+        for (int i = 0; i < NR; ++i) dma16s(lv + i * 1024, base, voff[i]);
+      } else {
+        // rows past Lk, or of an out-of-range entry, are zeros (their
+        // probabilities are zero, and 0 x inf must not reach the sums)
+        int ln = lane;
+        asm volatile("" : "+v"(ln));               // keep this rare path's offsets out of the loop preheader
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+          const int r = RPR * (wave * NR + i) + (ln >> LCPR);
+          const uint16_t* row = key0 >= 0 && r < a.Lk - key0 ? vp + (int64_t)(key0 + r) * a.v_sl
+                                                             : reinterpret_cast<const uint16_t*>(kZeroRow);
+          dma16(lv + i * 1024, row + ((ln & SWM) ^ v_swz<D>(r)) * 8);
+        }
+      }
+    } else {
+      const uint16_t* base = vp + max(key0, 0);    // V^T is zero padded to Lp
+#pragma unroll
+      for (int i = 0; i < NR; ++i) dma16s(lv + i * 1024, base, voff[i]);
+    }
   };
 
   // MFMA operand addressing.  A lane reads row l32 of a group of 32 rows and
@@ -530,6 +580,19 @@ void bsattn_kernel(AttnKArgs a) {
       TK == 128 ? lane_off_vr
                 : (uint32_t)((l32 >> 1) * 256 + (((((l32 & 1) << 3) | hi) ^ (l32 >> 1)) << 4));
   constexpr int VROW = TK == 128 ? 32 * 256 : 16 * 256;   // bytes per 32 d rows of V^T
+  // VD: each group of 16 lanes of a transposing read takes 4 keys x 16 dims,
+  // lane e of it supplying the address of key e / 4, dims 4 (e % 4) .. + 3, and
+  // receiving dim e of the 4 keys.  Two reads, of keys 4 hi .. + 3 and 8 + 4 hi
+  // .. + 3 of a 16-key group, give the lane's A operand in the key order in
+  // which the S^T accumulator holds P.  The operand of dims 32 dt .. + 31 is at
+  // the lane's offset with dt << 6 XORed in: v_swz moves the 64-byte pieces of a
+  // row, so that the 32 lanes of a phase (4 keys x 64 bytes) cover every bank once.
+  uint32_t lane_off_vd = 0;
+  if constexpr (VD) {
+    const int vrow = hi * 4 + ((lane & 15) >> 2);
+    lane_off_vd = (uint32_t)(vrow * ROWB + (lane & 1) * 8 +
+                             (((((lane >> 4) & 1) * 2 + ((lane & 3) >> 1)) ^ v_swz<D>(vrow)) << 4));
+  }
 
   // Running max (per query row) is kept in the exp2 domain of raw scores
   // times sc; it is only raised (and O rescaled) when a new score exceeds it
@@ -664,6 +727,17 @@ void bsattn_kernel(AttnKArgs a) {
   // O^T += V^T P^T for the V^T tile in buffer vbuf
   auto pv_mma = [&](int vbuf, const V8* pb) {
     const char* vt_base = reinterpret_cast<const char*>(lds[1][vbuf]);
+    if constexpr (VD) {
+#pragma unroll
+      for (int kk = 0; kk < C::KH / 16; ++kk)
+#pragma unroll
+        for (int dt = 0; dt < D / 32; ++dt) {
+          const uint32_t lo = (lane_off_vd ^ (uint32_t)(dt << 6)) + (kbase + kk * 16) * ROWB;
+          const V8 va = __builtin_bit_cast(V8, join8(lds_tr8(vt_base, lo), lds_tr8(vt_base, lo + 8 * ROWB)));
+          o[dt] = Ops::mma(va, pb[kk], o[dt]);
+        }
+      return;
+    }
 #pragma unroll
     for (int kk = 0; kk < C::KH / 16; ++kk) {
       const uint32_t lo = lane_off_v ^ (uint32_t)(((kbase >> 3) + 2 * kk) << 4);
@@ -739,14 +813,15 @@ void bsattn_kernel(AttnKArgs a) {
       // would hold its exponentials until the last one), the LDS operand
       // reads running six MFMAs ahead (measured best of 2 .. 8; three VALU
       // per MFMA against two: C2 -2.4%, C3a -4.6%, C3b -1.5%).
-      constexpr int NM = C::KT * (D / 16) + (C::KH / 16) * (D / 32);
+      constexpr int NS = C::KT * (D / 16), NM = NS + (C::KH / 16) * (D / 32);
       constexpr int LA = 6;
       constexpr int VPM = 3;
       __builtin_amdgcn_sched_group_barrier(0x100, LA, 0);        // DS reads
 #pragma unroll
       for (int i = 0; i < NM; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);       // MFMA
-        if (i + LA < NM) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        if (i + LA < (VD ? NS : NM)) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        else if (i + LA < NM) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);   // VD: a V operand is two reads
         __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);     // VALU
       }
     }
@@ -887,6 +962,8 @@ constexpr int kOrderThreads = 1024;
 constexpr int kTicketCounters = 9;               // 8 XCD shares + the shared pool
 constexpr int kPoolPercent = 10;                 // share of the work units (the shortest) in the shared pool
 constexpr int kOrderMaxBins = 8192;
+constexpr int64_t kDirectMaxKeys = 49152;        // see v_direct
+constexpr int64_t kDirectMaxKeysDense = 24576;
 constexpr int kOrderKeysPerThread = 8;           // keys kept in registers between the two passes
 // kvmajor = 0: one longest-first order over all units (the KV group left out of the key).
 __global__ __launch_bounds__(kOrderThreads) void order_kernel(const int32_t* __restrict__ cnt, int Hq, int Hk,
@@ -1065,7 +1142,23 @@ static int kv_major(const fs_attn_args& a, int Nq) {
   return per_group >= 4 * 2 * (int64_t)n ? 1 : 0;
 }
 
+// V is read as it is (no V^T pre-pass) where V is used few times: the pre-pass
+// moves V twice and is a launch (6 us at 1000 tokens, 26 us at 8192 with 32 KV
+// heads), the direct loop takes 1-3% longer, so the line is at a count of query
+// heads per KV head x keys.  Whole calls, V^T against direct, bf16, D = 128:
+//   dense  1000 tokens, 32 / 8 heads (4000): 29.5 / 23.6 us; 4096 (16384): 164 / 158;
+//          8192 (32768): 552 / 554; 16384 (65536): 2054 / 2067;
+//   lists  (density 0.3) 4096 (16384): 111 / 106 us; 8192 (32768): 229 / 224;
+//          32768 with 32 / 32 heads (32768): 2557 / 2513; block 64, 8192 with
+//          28 / 4 (57344): 213 / 209; 16384 (65536): 698 / 698, at D = 64 442 / 451.
+static bool v_direct(const fs_attn_args& a) {
+  if (a.blk_cnt != nullptr && a.bs < 64) return false;   // union mode
+  if (a.v_sl >= (1 << 23)) return false;                 // 32-bit lane offsets
+  return (int64_t)(a.Hq / a.Hk) * a.Lk <= (a.blk_cnt != nullptr ? kDirectMaxKeys : kDirectMaxKeysDense);
+}
+
 static size_t vt_bytes(const fs_attn_args& a) {
+  if (v_direct(a)) return 0;
   const int Nk = (a.Lk + a.bs - 1) / a.bs;
   return ((size_t)a.B * a.Hk * a.D * vt_len(Nk, a.bs) * 2 + 255) & ~(size_t)255;
 }
@@ -1092,6 +1185,16 @@ static int32_t* ticket_counters(const fs_attn_args& a) {
                                     align256((size_t)a.Hq * Nq * sizeof(int32_t)));
 }
 static bool union_mode(const fs_attn_args& a) { return a.blk_cnt != nullptr && a.bs < 64; }
+// Dense calls of few workgroups take 64 queries each instead of 128, so that
+// twice as many are in flight and a tile's keys are shared by two waves (the last
+// query block's chain of tiles is what such a call waits for).  128 against 64,
+// V direct, 32 / 8 heads: 1000 tokens (256 workgroups) 23.6 / 19.1 us, 2 x 768
+// (384) 27.0 / 22.7, 2048 (512) 53.4 / 50.2, 4 x 512 (512) 24.3 / 27.6, 4 x 1200
+// (1280) 74.5 / 80.4.
+static bool dense_by_64(const fs_attn_args& a, int Nq128) {
+  const int64_t wg = (int64_t)a.B * a.Hq * Nq128;
+  return wg <= 384 || (wg <= 512 && a.Lk >= 960);
+}
 static int union_groups(const fs_attn_args& a) {
   const int Nq = (a.Lq + a.bs - 1) / a.bs;
   const int R = 128 / a.bs;
@@ -1099,10 +1202,9 @@ static int union_groups(const fs_attn_args& a) {
 }
 
 // order pass (block lists only) and the main kernel, reading V^T from the workspace
-template <int BS, int TK, typename T, int D>
+template <int BS, int TK, typename T, int D, bool VD>
 static int launch_run(const fs_attn_args& a, int Nq, int Nk, hipStream_t s, int Lp = 0) {
   if (Lp == 0) Lp = vt_len(Nk, BS);                // else: V^T laid out for another block size
-  const uint16_t* vt = static_cast<const uint16_t*>(a.work);
   int32_t* order = nullptr;
   int32_t* ctr = nullptr;
   int static_units = 0, pool_units = 0;
@@ -1129,7 +1231,8 @@ static int launch_run(const fs_attn_args& a, int Nq, int Nk, hipStream_t s, int 
   AttnKArgs k;
   k.q = static_cast<const uint16_t*>(a.q);
   k.k = static_cast<const uint16_t*>(a.k);
-  k.vt = vt;
+  k.v = VD ? static_cast<const uint16_t*>(a.v) : static_cast<const uint16_t*>(a.work);
+  k.v_sb = a.v_sb; k.v_sh = a.v_sh; k.v_sl = VD ? (int)a.v_sl : 0;
   k.out = static_cast<uint16_t*>(a.out);
   k.blk_cnt = a.blk_cnt;
   k.blk_bits = a.blk_bits;
@@ -1145,7 +1248,7 @@ static int launch_run(const fs_attn_args& a, int Nq, int Nk, hipStream_t s, int 
   k.ctr = ctr;
   k.static_units = static_units;
   k.pool_units = pool_units;
-  bsattn_kernel<BS, TK, T, BS, D><<<grid, AttnCfg<BS, TK, D>::NT, 0, s>>>(k);
+  bsattn_kernel<BS, TK, T, BS, D, VD><<<grid, AttnCfg<BS, TK, D>::NT, 0, s>>>(k);
   return fs_host::launch_status("fs_bsattn");
 }
 
@@ -1174,7 +1277,8 @@ static int launch_run_union(const fs_attn_args& a, hipStream_t s) {
   AttnKArgs k;
   k.q = static_cast<const uint16_t*>(a.q);
   k.k = static_cast<const uint16_t*>(a.k);
-  k.vt = static_cast<const uint16_t*>(a.work);
+  k.v = static_cast<const uint16_t*>(a.work);
+  k.v_sb = k.v_sh = k.v_sl = 0;
   k.out = static_cast<uint16_t*>(a.out);
   k.blk_cnt = u_cnt;
   k.blk_bits = nullptr;
@@ -1199,7 +1303,7 @@ using namespace fs;
 
 extern "C" size_t fs_bsattn_work_bytes(const fs_attn_args* a) {
   if (!a || a->B <= 0 || a->Hq <= 0 || a->Hk <= 0 || a->Lq <= 0 || a->Lk <= 0 || a->D <= 0 || a->bs <= 0) return 0;
-  size_t n = vt_bytes(*a) + order_bytes(*a);
+  size_t n = vt_bytes(*a) + order_bytes(*a);       // never 0
   if (union_mode(*a)) {
     const size_t Ng = (size_t)union_groups(*a), Nk = (size_t)(a->Lk + a->bs - 1) / a->bs;
     n += align256((size_t)a->Hq * Ng * sizeof(int32_t)) + (size_t)a->Hq * Ng * Nk * sizeof(uint32_t);
@@ -1245,6 +1349,7 @@ static int check_attn(const fs_attn_args* a, const char* fn) {
 
 extern "C" int fs_bsattn_prepare(const fs_attn_args* a, void* stream) {
   if (int rc = check_attn(a, "fs_bsattn_prepare")) return rc;
+  if (v_direct(*a)) return FS_OK;                  // V is read as it is
   const int Nk = (a->Lk + a->bs - 1) / a->bs;
   const int Lp = vt_len(Nk, a->bs);
   auto vt = a->D == 64 ? vt_kernel<64> : vt_kernel<128>;
@@ -1255,20 +1360,21 @@ extern "C" int fs_bsattn_prepare(const fs_attn_args* a, void* stream) {
 }
 
 // head dim D, element type T: the kernels of one call
-template <typename T, int D>
+template <typename T, int D, bool VD>
 static int run_typed(const fs_attn_args* a, int Nq, int Nk, hipStream_t s) {
-  if (a->bs == 128) return launch_run<128, 64, T, D>(*a, Nq, Nk, s);
-  if (a->bs < 64) {
-    if (a->blk_cnt) {
-      // 16- and 32-token lists: unions over groups of 128 queries
-      return a->bs == 32 ? launch_run_union<32, T, D>(*a, s) : launch_run_union<16, T, D>(*a, s);
-    }
-    // dense causal attention does not depend on the block size: the 128-token
-    // kernel, reading V^T as it was laid out for this block size
-    const int Nq128 = (a->Lq + 127) / 128, Nk128 = (a->Lk + 127) / 128;
-    return launch_run<128, 64, T, D>(*a, Nq128, Nk128, s, vt_len(Nk, a->bs));
-  }
-  return launch_run<64, 64, T, D>(*a, Nq, Nk, s);
+  if (a->blk_cnt) return a->bs == 128 ? launch_run<128, 64, T, D, VD>(*a, Nq, Nk, s) : launch_run<64, 64, T, D, VD>(*a, Nq, Nk, s);
+  // Dense attention does not depend on the block size, only the workgroups'
+  // queries do.  Lp: V^T as it was laid out for the call's block size.
+  const int Lp = vt_len(Nk, a->bs);
+  const int Nq128 = (a->Lq + 127) / 128, Nk128 = (a->Lk + 127) / 128;
+  if (a->bs == 64 || dense_by_64(*a, Nq128)) return launch_run<64, 64, T, D, VD>(*a, (a->Lq + 63) / 64, (a->Lk + 63) / 64, s, Lp);
+  return launch_run<128, 64, T, D, VD>(*a, Nq128, Nk128, s, Lp);
+}
+template <typename T, int D>
+static int run_head(const fs_attn_args* a, int Nq, int Nk, hipStream_t s) {
+  // 16- and 32-token lists: unions over groups of 128 queries
+  if (union_mode(*a)) return a->bs == 32 ? launch_run_union<32, T, D>(*a, s) : launch_run_union<16, T, D>(*a, s);
+  return v_direct(*a) ? run_typed<T, D, true>(a, Nq, Nk, s) : run_typed<T, D, false>(a, Nq, Nk, s);
 }
 
 extern "C" int fs_bsattn_run(const fs_attn_args* a, void* stream) {
@@ -1277,8 +1383,8 @@ extern "C" int fs_bsattn_run(const fs_attn_args* a, void* stream) {
   const int Nk = (a->Lk + a->bs - 1) / a->bs;
   hipStream_t s = (hipStream_t)stream;
   if (a->D == 64)
-    return a->dtype == FS_DTYPE_BF16 ? run_typed<bf16_t, 64>(a, Nq, Nk, s) : run_typed<f16_t, 64>(a, Nq, Nk, s);
-  return a->dtype == FS_DTYPE_BF16 ? run_typed<bf16_t, 128>(a, Nq, Nk, s) : run_typed<f16_t, 128>(a, Nq, Nk, s);
+    return a->dtype == FS_DTYPE_BF16 ? run_head<bf16_t, 64>(a, Nq, Nk, s) : run_head<f16_t, 64>(a, Nq, Nk, s);
+  return a->dtype == FS_DTYPE_BF16 ? run_head<bf16_t, 128>(a, Nq, Nk, s) : run_head<f16_t, 128>(a, Nq, Nk, s);
 }
 
 extern "C" int fs_bsattn(const fs_attn_args* a, void* stream) {

@@ -348,7 +348,7 @@ FS_API int fs_flex(const fs_flex_args* a, void* stream);
  * are attended 128 queries at a time over the union of 128 / bs rows,
  * up to 8192 key blocks).  All tensors are
  * strided views with d contiguous.
- * work: fs_bsattn_work_bytes(a) bytes of device scratch (V is staged there
+ * work: fs_bsattn_work_bytes(a) bytes of device scratch (V may be staged there
  * transposed, and the work items' longest-first order and the counters from
  * which the attention kernel's workgroups take their work items are formed
  * there, before the attention kernel runs).  Calls that overlap on one
@@ -371,11 +371,14 @@ FS_API size_t fs_bsattn_work_bytes(const fs_attn_args* a);
 /* The whole stage-2 call: fs_bsattn_prepare then fs_bsattn_run. */
 FS_API int fs_bsattn(const fs_attn_args* a, void* stream);
 /* The two halves of fs_bsattn, for callers that time or reuse them apart.
- * prepare: writes V^T of every KV head into work (depends on v, and on bs
- * and whether block lists are given: 16- and 32-token lists take V^T block
- * by block).  run: the longest-first order pass (block lists only) and the
- * attention kernel; reads V^T from work, so a prepare with the same v, Lk,
- * bs, lists (present or not) and work must precede it on the stream.  Both replace the same reference call as
+ * prepare: writes V^T of every KV head into work where the call reads it from
+ * there (depends on v, and on bs and whether block lists are given: 16- and
+ * 32-token lists take V^T block by block); a call that uses V few times (a
+ * short sequence, few query heads per KV head) reads v itself and prepare does
+ * nothing.  run: the longest-first order pass (block lists only) and the
+ * attention kernel; reads V^T from work, or v, so a prepare with the same v, Lk,
+ * bs, lists (present or not) and work must precede it on the stream, and v
+ * must stay as it was.  Both replace the same reference call as
  * fs_bsattn (my_attn_v7.py:775-786). */
 FS_API int fs_bsattn_prepare(const fs_attn_args* a, void* stream);
 FS_API int fs_bsattn_run(const fs_attn_args* a, void* stream);
