@@ -257,7 +257,11 @@ void bsattn_kernel(AttnKArgs a) {
   using C = AttnCfg<BS, TK, D>;
   static_assert(D == 64 || D == 128, "head dim 64 or 128");
   // K tiles: rows of D * 2 bytes, CPR 16-byte chunks each, chunk c of row r
-  // stored at c ^ (r & SWM); a 1 KiB copy region holds RPR rows
+  // stored at c ^ (r & SWM), at D = 64 at c ^ ((r >> 1) & SWM); a 1 KiB copy
+  // region holds RPR rows.  The 16 lanes of an operand read phase (one row each)
+  // then hit distinct banks: at D = 64 two rows share a 256-byte bank span, and
+  // the row's bit 0 separates them already (with r & SWM there, rows r and r + 8
+  // collided, a third of the LDS cycles of a D = 64 call).
   constexpr int ROWB = D * 2, CPR = D / 8, SWM = CPR - 1, RPR = 1024 / ROWB, LCPR = D == 128 ? 4 : 3;
   constexpr bool UNION = LB < BS;
   constexpr int EPT = UNION ? TK / LB : 1;         // union entries per tile
@@ -447,7 +451,7 @@ void bsattn_kernel(AttnKArgs a) {
     int rk = r, ck = c;                            // K: rows RPR R .. RPR R + RPR - 1
     if constexpr (D != 128) {
       rk = RPR * R + (lane >> LCPR);
-      ck = (lane & SWM) ^ (rk & SWM);
+      ck = (lane & SWM) ^ ((rk >> 1) & SWM);
     }
     if constexpr (UNION) {
       // K rows relative to this wave's 16 rows of the tile; V^T: the key
@@ -492,7 +496,8 @@ void bsattn_kernel(AttnKArgs a) {
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
           const int rr = RPR * i + (ln >> LCPR);     // row within this wave's block
-          const int c = (ln & SWM) ^ ((RPR * (wave * NR + i) + (ln >> LCPR)) & SWM);
+          const int rt = RPR * (wave * NR + i) + (ln >> LCPR);
+          const int c = (ln & SWM) ^ ((D == 128 ? rt : rt >> 1) & SWM);
           dma16s(lk + i * 1024, base, (uint32_t)(min(rr, a.Lk - 1 - kc) * a.k_sl + c * 8) * 2u);
         }
       }
@@ -512,7 +517,7 @@ void bsattn_kernel(AttnKArgs a) {
 #pragma unroll
       for (int i = 0; i < NR; ++i) {
         const int r = RPR * (wave * NR + i) + (ln >> LCPR);
-        const int c = (ln & SWM) ^ (r & SWM);
+        const int c = (ln & SWM) ^ ((D == 128 ? r : r >> 1) & SWM);
         dma16s(lk + i * 1024, base, (uint32_t)(min(r, a.Lk - 1 - kc) * a.k_sl + c * 8) * 2u);
       }
     }
@@ -574,7 +579,7 @@ void bsattn_kernel(AttnKArgs a) {
   // For V^T tiles of 64 keys an LDS row holds two d rows (d = 2 r + (chunk >> 3)):
   // the lane's d row dt * 32 + l32 sits in LDS row dt * 16 + (l32 >> 1), chunk
   // (l32 & 1) * 8 + C0 + hi.
-  const uint32_t lane_off = (uint32_t)(l32 * ROWB + ((hi ^ (l32 & SWM)) << 4));   // K tile rows
+  const uint32_t lane_off = (uint32_t)(l32 * ROWB + ((hi ^ ((D == 128 ? l32 : l32 >> 1) & SWM)) << 4));   // K tile rows
   const uint32_t lane_off_vr = (uint32_t)(l32 * 256 + ((hi ^ (l32 & 15)) << 4));   // 256-byte V^T rows
   const uint32_t lane_off_v =
       TK == 128 ? lane_off_vr
