@@ -609,7 +609,10 @@ void bsattn_kernel(AttnKArgs a) {
   // sum exceeds 2^64 (or is inf / nan, as on a row's first tile) is redone
   // with the raised max.  Against the row max: C3a -4.6%; at block 128 (32
   // MFMAs per wave) the row max is kept, the other form measured 3.5% slower.
-  constexpr bool kRowMax = C::KG == 1;
+  // At D = 64 a score costs the same softmax work beside half the MFMAs, the
+  // loop is bound by it, and the row max goes there too (block 128, 32 / 8
+  // heads: 8192 tokens 145.5 -> 136 us, 65536 4942 -> 4680).
+  constexpr bool kRowMax = C::KG == 1 && D == 128;
   float m_run = -INFINITY, l_run = 0.f;
   f32x16_t o[D / 32];
 #pragma unroll

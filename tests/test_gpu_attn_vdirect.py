@@ -59,3 +59,30 @@ def test_dense_by_64_queries(L, B):
     s.masked_fill_(torch.ones(L, L, dtype=torch.bool).triu(1), float("-inf"))
     ref = (torch.softmax(s, -1) @ vf).transpose(1, 2)
     assert (o - ref).abs().max() < 2e-2
+
+
+@pytest.mark.parametrize("growth", [30.0, 3000.0, -3000.0])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Hq", [2, 32])
+def test_head_dim_64_running_max(growth, dtype, Hq):
+    """Head dim 64 takes its exponentials against the running max with no row
+    max: scores that rise or fall along the keys, far past the range of a 16-bit
+    probability, direct (2 heads) and through V^T (32 heads on one KV head)."""
+    L, D = 1600, 64
+    g = torch.Generator().manual_seed(12)
+    u = torch.randn(D, generator=g)
+    u /= u.norm()
+    q = torch.randn(1, Hq, L, D, generator=g) + 10.0 * u
+    k = torch.randn(1, 1, L, D, generator=g) + (torch.arange(L, dtype=torch.float32) / L * growth)[:, None] * u
+    v = torch.randn(1, 1, L, D, generator=g)
+    q, k, v = (x.to(dtype) for x in (q, k, v))
+    s = (q.float() @ k.float().transpose(-1, -2)) * D ** -0.5
+    s.masked_fill_(torch.ones(L, L, dtype=torch.bool).triu(1), float("-inf"))
+    ref = (torch.softmax(s, -1) @ v.float()).transpose(1, 2)
+    qd, kd, vd = (x.to(DEV) for x in (q, k, v))
+    assert (block_sparse_attention(qd, kd, vd).float().cpu() - ref).abs().max() < 2e-2
+    for bs in (128, 64, 32):
+        n = -(-L // bs)
+        mask = torch.ones(Hq, n, n, dtype=torch.bool).tril()
+        cnt, bits = (t.to(DEV) for t in bits_from_mask(mask))
+        assert (block_sparse_attention(qd, kd, vd, cnt, bits, block_size=bs).float().cpu() - ref).abs().max() < 2e-2
