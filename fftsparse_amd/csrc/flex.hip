@@ -38,7 +38,8 @@
 //                 bit masks.
 // flex_cover_rows_kernel: for each sparse head, the block-level causal
 //   attention softmax(avg_q / sqrt(D) avg_k^T) (block means of q, the last one
-//   rescaled to its real rows); its cut at gamma * N by cut_pass_kernel, and
+//   rescaled to its real rows; the part up to the diagonal, the rest is left
+//   unwritten and unread); its cut at gamma * N by cut_pass_kernel, and
 //   flex_cover_emit_kernel writes the kept entries as an N x N bit mask.
 // flex_lists_kernel: per (head, block row r): the vertical columns <= r, the
 //   diagonals r - s of the chosen slash offsets, the sparse cover's row, as an
@@ -475,7 +476,9 @@ __device__ CutResult radix_topk(const float* x, int n, int want, CutScratch* cs)
 // ballot per word, no atomics).  Each wave owns a contiguous range of words;
 // when the cut splits the elements equal to its key, a fixed-order prefix of
 // the waves' tie counts ranks them.
-// Words wb .. we-1 only, with base_rank ties before them, when given.
+// Words wb .. we-1 only, with base_rank ties before them, when given.  TRI: x
+// holds the elements up to the diagonal only, the others are not in the cut.
+template <bool TRI = false>
 __device__ void emit_cut(const float* x, int rows, int row_len, const CutResult& cut, uint64_t* out, int* scan,
                          int wb = 0, int we = -1, int base_rank = 0) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -491,7 +494,7 @@ __device__ void emit_cut(const float* x, int rows, int row_len, const CutResult&
     int cnt = 0;
     for (int w = w0; w < w1; ++w) {
       const int r = w / wpr, c = (w - r * wpr) * 64 + lane;
-      const bool eq = c < row_len && order_key(x[(int64_t)r * row_len + c]) == cut.key;
+      const bool eq = c < (TRI ? r + 1 : row_len) && order_key(x[(int64_t)r * row_len + c]) == cut.key;
       cnt += __popcll(__ballot(eq));
     }
     if (lane == 0) scan[wave] = cnt;
@@ -502,7 +505,7 @@ __device__ void emit_cut(const float* x, int rows, int row_len, const CutResult&
   for (int w = w0; w < w1; ++w) {
     const int r = w / wpr, c = (w - r * wpr) * 64 + lane;
     bool in = false, eq = false;
-    if (c < row_len) {
+    if (c < (TRI ? r + 1 : row_len)) {
       const uint32_t k = order_key(x[(int64_t)r * row_len + c]);
       in = k > cut.key;
       eq = k == cut.key;
@@ -533,6 +536,7 @@ struct CutJobs {
   const float* x1;              // kind 1 data (kinds == 2)
   int64_t stride;
   int n;                        // elements per job
+  int tri;                      // rows of a lower triangle [tri][tri] (0: n elements in a row); only that part is read
   int kinds;                    // jobs per head (1 or 2)
   int jobs, slices;
   int scale_exp;                // masses as integers x * 2^scale_exp
@@ -654,14 +658,11 @@ __global__ __launch_bounds__(kCutSliceThreads) void cut_pass_kernel(CutJobs c) {
   }
   __syncthreads();
   const float* x = job_data(c, j);
-  const int per = (c.n + c.slices - 1) / c.slices;
-  const int i0 = sl * per, i1 = min(c.n, i0 + per);
   const double sc = ldexp(1.0, c.scale_exp);
   constexpr int shift = 24 - 8 * PASS;
   const uint32_t prefix = st.prefix;
   const int copy = tid % kCutCopies;
-  for (int i = i0 + tid; i < i1; i += kCutSliceThreads) {
-    const float v = x[i];
+  auto add = [&](float v) {
     const uint32_t key = order_key(v);
     if (PASS == 0 || (key >> (shift + 8)) == prefix) {
       const uint32_t d = (key >> shift) & 255u;
@@ -669,6 +670,27 @@ __global__ __launch_bounds__(kCutSliceThreads) void cut_pass_kernel(CutJobs c) {
       if (m) atomicAdd(reinterpret_cast<unsigned long long*>(&lhm[copy][d]), (unsigned long long)m);
       atomicAdd(&lhc[copy][d], 1u);
     }
+  };
+  if (c.tri) {
+    // a wave per row, rows dealt over the job's waves; what lies above the
+    // diagonal is zero (no mass, so it moves no cut) and is left out
+    const int lane = tid & 63, nw = c.slices * (kCutSliceThreads / 64);
+    for (int r = sl * (kCutSliceThreads / 64) + __builtin_amdgcn_readfirstlane(tid >> 6); r < c.tri; r += nw) {
+      const float* xr = x + (int64_t)r * c.tri;
+      int i = lane;
+      for (; i + 192 <= r; i += 256) {             // four loads in flight
+        const float v0 = xr[i], v1 = xr[i + 64], v2 = xr[i + 128], v3 = xr[i + 192];
+        add(v0);
+        add(v1);
+        add(v2);
+        add(v3);
+      }
+      for (; i <= r; i += 64) add(xr[i]);
+    }
+  } else {
+    const int per = (c.n + c.slices - 1) / c.slices;
+    const int i0 = sl * per, i1 = min(c.n, i0 + per);
+    for (int i = i0 + tid; i < i1; i += kCutSliceThreads) add(x[i]);
   }
   __syncthreads();
   uint64_t* hm = c.hm + ((int64_t)PASS * c.jobs + j) * 256;
@@ -859,134 +881,152 @@ struct FlexCoverK {
   float sqrt_d, gamma;
 };
 
-// block-level causal attention rows of a sparse head: one workgroup per (head,
-// kCoverRows consecutive block rows).  The K block means are staged in LDS 256
-// rows at a time (row stride 260 bytes: thread t reads row t, bank (t + d / 2)
-// % 64, conflict-free) and each staged row serves all the workgroup's query
-// rows.  Per row, as one row per workgroup would: the score of key block j is
-// the fp32 sum over d in order, rounded to T; thread t takes the blocks j = t,
-// t + 256, ... (its exponential sums in that order), the maxima and sums are
-// reduced by the same tree, and the scores and their exponentials pass
-// through the row's place in attn.
-constexpr int kCoverRows = 8;
-constexpr int kCoverStride = kFD + 2;            // staged row: 130 bf16 = 260 bytes
+// block-level causal attention rows of a sparse head: one workgroup (4 waves)
+// per (head, 32 consecutive block rows).  The rows' Q block means are the B
+// operand of v_mfma_f32_32x32x16 (32 keys x 32 rows, scores rounded to T), wave w
+// taking the key tiles w, w + 4, ..; the tiles are formed twice, first for each
+// row's maximum and sum of exponentials (per lane online, merged over the lanes
+// and waves of the row), then for the probabilities, of which only the causal
+// part of a row is written.  What bounds it: the read of the sparse heads' Q (201
+// MB for 24 heads of 32768 tokens, 40 us at 5 TB/s) and two exponentials per
+// score.  Those heads at 32-token blocks: 92 us, against 440 with scalar dot
+// products over K block means staged in LDS, 8 rows per workgroup, 2-byte Q loads
+// and the scores passing through memory.
+constexpr int kCoverRows = 32;
+constexpr int kCoverStride = kFD + 8;            // staged row: 136 values, 16-byte chunks spread over the banks
 template <typename T>
 __global__ __launch_bounds__(kFThreads) void flex_cover_rows_kernel(FlexCoverK a) {
-  __shared__ float aq[kCoverRows][kFD];
-  __shared__ __attribute__((aligned(16))) uint16_t kst[kFThreads * kCoverStride];
-  __shared__ float red[kFThreads];
+  __shared__ __attribute__((aligned(16))) uint16_t aq[kCoverRows * kCoverStride];
+  __shared__ float red[kFThreads][2];
   // a head's workgroups in order of decreasing row (the longest rows start
   // first); consecutive workgroups (one head's) fall on different XCDs
   const int ngr = (a.nb + kCoverRows - 1) / kCoverRows;
   const int h = blockIdx.x / ngr, i0 = (ngr - 1 - (int)(blockIdx.x % ngr)) * kCoverRows;
   if (a.info[h * 4 + 2] == 0) return;              // not a sparse head
   const int tid = threadIdx.x, bs = a.bs, nb = a.nb, L = a.L;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hi = lane >> 5;
   const int nr = min(kCoverRows, nb - i0);         // rows of this workgroup
   const int kvh = kv_head(h, a.Hq, a.Hk, a.gqa_interleave);
   const int pad = nb * bs - L;
   // block means of q over bs rows (zero padded), in T; the last block rescaled
   // as (mean * bs) / (bs - pad), each step rounded to T.  Thread t forms the
-  // means of dim t % 128 for rows t / 128, t / 128 + 2, ...; the loads of 8
-  // tokens of every such row are issued before they are added (in token order).
+  // means of dims 8 (t % 16) .. + 7 for rows t / 16 and t / 16 + 16; the loads of
+  // 8 tokens are issued before they are added (in token order).
   {
-    constexpr int kPer = kCoverRows * kFD / kFThreads;   // (row, dim) pairs per thread
-    const uint16_t* qh = a.q + (int64_t)h * a.q_sh;
-    const int d = tid % kFD, rr0 = tid / kFD;
-    float sum[kPer];
+    const uint16_t* qh = a.q + (int64_t)h * a.q_sh + (tid & 15) * 8;
+    for (int rr = tid >> 4; rr < kCoverRows; rr += kFThreads / 16) {
+      const int t0 = (i0 + rr) * bs;
+      float sum[8];
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) sum[u] = 0.f;
-    for (int r0 = 0; r0 < bs; r0 += 8) {
-      float x[kPer][8];
+      for (int e = 0; e < 8; ++e) sum[e] = 0.f;
+      for (int r0 = 0; r0 < bs; r0 += 8) {
+        uint4 x[8];
 #pragma unroll
-      for (int u = 0; u < kPer; ++u)
+        for (int r = 0; r < 8; ++r)
+          x[r] = *reinterpret_cast<const uint4*>(qh + (int64_t)min(t0 + r0 + r, L - 1) * a.q_sl);
 #pragma unroll
         for (int r = 0; r < 8; ++r) {
-          const int i = i0 + rr0 + 2 * u, t = i * bs + r0 + r;
-          x[u][r] = (rr0 + 2 * u < nr && t < L) ? to_f32(T{qh[(int64_t)t * a.q_sl + d]}) : 0.f;
-        }
+          const uint32_t w[4] = {x[r].x, x[r].y, x[r].z, x[r].w};
+          const bool in = t0 + r0 + r < L;
 #pragma unroll
-      for (int u = 0; u < kPer; ++u)
-#pragma unroll
-        for (int r = 0; r < 8; ++r) sum[u] += x[u][r];
-    }
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      const int rr = rr0 + 2 * u, i = i0 + rr;
-      if (rr >= nr) continue;
-      float m = Conv<T>::round(sum[u] / (float)bs);
-      if (pad && i == nb - 1) m = Conv<T>::round(Conv<T>::round(m * (float)bs) / (float)(bs - pad));
-      aq[rr][d] = Conv<T>::round(m / a.sqrt_d);
-    }
-  }
-  const int last = i0 + nr - 1;                    // the workgroup's last row: keys 0 .. last
-  float mx[kCoverRows];
-#pragma unroll
-  for (int rr = 0; rr < kCoverRows; ++rr) mx[rr] = -INFINITY;
-  float* rows = a.attn + ((int64_t)h * nb + i0) * nb;
-  const uint16_t* kbase = a.avg_k + (int64_t)kvh * nb * kFD;
-  for (int j0 = 0; j0 <= last; j0 += kFThreads) {
-    __syncthreads();                               // aq written / the previous tile consumed
-    // stage rows j0 .. j0 + 255 (16-byte global loads, 4-byte LDS writes)
-    for (int c = tid; c < kFThreads * (kFD / 8); c += kFThreads) {
-      const int r = c / (kFD / 8), cc = c - r * (kFD / 8);
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (j0 + r <= last) v = *reinterpret_cast<const uint4*>(kbase + (int64_t)(j0 + r) * kFD + cc * 8);
-      uint32_t* dst = reinterpret_cast<uint32_t*>(kst + r * kCoverStride + cc * 8);
-      dst[0] = v.x; dst[1] = v.y; dst[2] = v.z; dst[3] = v.w;
-    }
-    __syncthreads();
-    const int j = j0 + tid;
-    if (j <= last) {
-      float acc[kCoverRows];
-#pragma unroll
-      for (int rr = 0; rr < kCoverRows; ++rr) acc[rr] = 0.f;
-      const uint32_t* kr = reinterpret_cast<const uint32_t*>(kst + tid * kCoverStride);
-      for (int d2 = 0; d2 < kFD / 2; ++d2) {
-        const uint32_t w = kr[d2];
-        const float k0 = to_f32(T{(uint16_t)(w & 0xffffu)}), k1 = to_f32(T{(uint16_t)(w >> 16)});
-#pragma unroll
-        for (int rr = 0; rr < kCoverRows; ++rr) {
-          acc[rr] += aq[rr][2 * d2] * k0;
-          acc[rr] += aq[rr][2 * d2 + 1] * k1;
+          for (int e = 0; e < 8; ++e) {
+            const float v = to_f32(T{(uint16_t)(w[e >> 1] >> (16 * (e & 1)))});
+            sum[e] += in ? v : 0.f;
+          }
         }
       }
+      uint32_t o[4];
 #pragma unroll
-      for (int rr = 0; rr < kCoverRows; ++rr) {
-        if (rr < nr && j <= i0 + rr) {
-          const float v = Conv<T>::round(acc[rr]);
-          rows[(int64_t)rr * nb + j] = v;
-          mx[rr] = fmaxf(mx[rr], v);
-        }
+      for (int e = 0; e < 8; ++e) {
+        float m = Conv<T>::round(sum[e] / (float)bs);
+        if (pad && i0 + rr == nb - 1) m = Conv<T>::round(Conv<T>::round(m * (float)bs) / (float)(bs - pad));
+        const uint32_t v = __builtin_bit_cast(uint16_t, Conv<T>::store(m / a.sqrt_d));
+        if (e & 1) o[e >> 1] |= v << 16;
+        else o[e >> 1] = v;
       }
+      *reinterpret_cast<uint4*>(aq + rr * kCoverStride + (tid & 15) * 8) = make_uint4(o[0], o[1], o[2], o[3]);
     }
   }
-  for (int rr = 0; rr < nr; ++rr) {
-    const int i = i0 + rr;
-    float* out = rows + (int64_t)rr * nb;
-    red[tid] = mx[rr];
-    __syncthreads();
-    for (int s = kFThreads / 2; s > 0; s >>= 1) {
-      if (tid < s) red[tid] = fmaxf(red[tid], red[tid + s]);
-      __syncthreads();
+  __syncthreads();
+  uint4 qf[kFD / 16];                              // row l32, dims st 16 + hi 8 .. + 7
+#pragma unroll
+  for (int st = 0; st < kFD / 16; ++st)
+    qf[st] = *reinterpret_cast<const uint4*>(aq + l32 * kCoverStride + st * 16 + hi * 8);
+  const int last = i0 + nr - 1, row = i0 + l32;    // the workgroup's last row: keys 0 .. last
+  const int ntile = last / 32 + 1;
+  const uint16_t* kbase = a.avg_k + (int64_t)kvh * nb * kFD + hi * 8;
+  auto load = [&](int t, uint4* kv) {
+    const uint16_t* kr = kbase + (int64_t)min(32 * t + l32, last) * kFD;
+#pragma unroll
+    for (int st = 0; st < kFD / 16; ++st) kv[st] = *reinterpret_cast<const uint4*>(kr + st * 16);
+  };
+  // scores of keys 32 t + (r / 4) 8 + hi 4 + r % 4, rounded to T
+  auto scores = [&](const uint4* kv, float* x) {
+    f32x16_t acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+#pragma unroll
+    for (int st = 0; st < kFD / 16; ++st) acc = FMma<T>::mma(kv[st], qf[st], acc);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) x[r] = Conv<T>::round(acc[r]);
+  };
+  auto seen = [&](int t, int r) { return 32 * t + (r >> 2) * 8 + hi * 4 + (r & 3) <= row; };
+  // the wave's tiles, the next one's keys loaded while one is worked on
+  auto tiles = [&](auto body) {
+    constexpr int W = kFThreads / 64;
+    uint4 k0[kFD / 16], k1[kFD / 16];
+    if (wave < ntile) load(wave, k0);
+    for (int t = wave; t < ntile; t += 2 * W) {
+      if (t + W < ntile) load(t + W, k1);
+      float x[16];
+      scores(k0, x);
+      body(t, x);
+      if (t + W >= ntile) break;
+      if (t + 2 * W < ntile) load(t + 2 * W, k0);
+      scores(k1, x);
+      body(t + W, x);
     }
-    const float m = red[0];
-    __syncthreads();
-    float se = 0.f;
-    for (int j = tid; j <= i; j += kFThreads) {
-      const float e = expf(out[j] - m);
-      out[j] = e;
-      se += e;
+  };
+  float m_run = -INFINITY, l_run = 0.f;
+  tiles([&](int t, const float* x) {
+    float mx = m_run;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mx = seen(t, r) ? fmaxf(mx, x[r]) : mx;
+    if (mx > -INFINITY) {
+      float se = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float e = expf(x[r] - mx);
+        se += seen(t, r) ? e : 0.f;
+      }
+      l_run = l_run * expf(m_run - mx) + se;
+      m_run = mx;
     }
-    red[tid] = se;
-    __syncthreads();
-    for (int s = kFThreads / 2; s > 0; s >>= 1) {
-      if (tid < s) red[tid] += red[tid + s];
-      __syncthreads();
+  });
+  // the row's lanes: l32 and l32 + 32 of the four waves, merged in that order by each of them
+  red[tid][0] = m_run;
+  red[tid][1] = l_run;
+  __syncthreads();
+  float m = -INFINITY, se = 0.f;
+  for (int e = l32; e < kFThreads; e += 32) m = fmaxf(m, red[e][0]);
+  for (int e = l32; e < kFThreads; e += 32) se += red[e][0] > -INFINITY ? red[e][1] * expf(red[e][0] - m) : 0.f;
+  float* out = a.attn + ((int64_t)h * nb + row) * nb;
+  tiles([&](int t, const float* x) {
+    float p[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) p[r] = expf(x[r] - m) / se;
+    if (l32 >= nr) return;
+    float* o = out + 32 * t + hi * 4;
+    if (32 * t + 31 <= i0 && (nb & 3) == 0) {      // a whole tile below the diagonal: 16-byte stores
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<float4*>(o + g * 8) = make_float4(p[4 * g], p[4 * g + 1], p[4 * g + 2], p[4 * g + 3]);
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (seen(t, r)) o[(r >> 2) * 8 + (r & 3)] = p[r];
     }
-    se = red[0];
-    __syncthreads();
-    for (int j = tid; j < nb; j += kFThreads) out[j] = j <= i ? out[j] / se : 0.f;
-  }
+  });
 }
 
 // the cover of gamma * N over a sparse head's N x N probabilities
@@ -1020,7 +1060,7 @@ __global__ __launch_bounds__(kFHeadThreads) void flex_cover_ties_kernel(FlexCove
   int cnt = 0;
   for (int w = wb + wave; w < we; w += kFHeadThreads / 64) {
     const int r = w / wpr, col = (w - r * wpr) * 64 + lane;
-    const bool eq = col < nb && order_key(x[(int64_t)r * nb + col]) == cut.key;
+    const bool eq = col <= r && order_key(x[(int64_t)r * nb + col]) == cut.key;
     cnt += __popcll(__ballot(eq));
   }
   if (lane == 0) wsum[wave] = cnt;
@@ -1048,14 +1088,14 @@ __global__ __launch_bounds__(kFHeadThreads) void flex_cover_emit_kernel(FlexCove
     for (int v = 0; v < sl; ++v) base += ties[h * c.slices + v];
     int wb, we;
     cover_slice_words(nb, c.slices, sl, &wb, &we);
-    emit_cut(x, nb, nb, cut, cov, scan, wb, we, base);
+    emit_cut<true>(x, nb, nb, cut, cov, scan, wb, we, base);
   } else {
     const int wpr = (nb + 63) >> 6, nwords = nb * wpr;
     const int step = c.slices * (kFHeadThreads / 64);
     for (int w = sl * (kFHeadThreads / 64) + (tid >> 6); w < nwords; w += step) {
       const int r = w / wpr, col = (w - r * wpr) * 64 + lane;
       bool in = false;
-      if (col < nb) {
+      if (col <= r) {
         const uint32_t k = order_key(x[(int64_t)r * nb + col]);
         in = k > cut.key || (k == cut.key && cut.take_eq > 0);
       }
@@ -1241,6 +1281,7 @@ static int launch_flex(const fs_flex_args& a, hipStream_t s) {
   cc.x1 = nullptr;
   cc.stride = (int64_t)nb * nb;
   cc.n = nb * nb;
+  cc.tri = nb;
   cc.kinds = 1;
   cc.jobs = a.Hq;
   cc.slices = std::max(1, std::min(256, (nb * nb + 16383) / 16384));
