@@ -53,7 +53,8 @@ namespace fs {
 constexpr int kFD = 128;
 constexpr int kFThreads = 256;
 constexpr int kFTile = 128;                      // key columns per tile
-constexpr int kFChunk = 2048;                    // key columns per workgroup
+constexpr int kFChunk = 2048;                    // most key columns per workgroup of the last-block passes
+constexpr int kFChunkMin = 512;
 constexpr int kFHeadThreads = 1024;
 constexpr int kFMaxBlocks = 8192;
 constexpr int kFWords = kFMaxBlocks / 64;
@@ -90,7 +91,7 @@ struct FlexK {
   const uint16_t* q;            // [Hq][L][D] view (strides q_sh, q_sl)
   const uint16_t* k;
   int64_t q_sh, q_sl, k_sh, k_sl;
-  int Hq, Hk, L, bs, nb, gqa_interleave, nchunk;
+  int Hq, Hk, L, bs, nb, gqa_interleave, nchunk, chunk;   // chunk: key columns per workgroup
   float sqrt_d;
   float* part;                  // [Hq][nchunk][bs][2] (max, sum) per chunk
   float* vert;                  // [Hq][L]
@@ -146,8 +147,8 @@ __global__ __launch_bounds__(kFThreads) void flex_lastq_kernel(FlexK a) {
     qf[st] = make_uint4(o[0], o[1], o[2], o[3]);
   }
 
-  const int c_begin = chunk * kFChunk;
-  const int c_end = min(L, c_begin + kFChunk);
+  const int c_begin = chunk * a.chunk;
+  const int c_end = min(L, c_begin + a.chunk);
   // PASS 2 starts one tile early (carry of the diagonals that cross into the chunk)
   const int t_first = (PASS == 2 && chunk > 0) ? c_begin - kFTile : c_begin;
   const int lim_causal = L - bs + row;            // the last block: key <= query
@@ -175,18 +176,25 @@ __global__ __launch_bounds__(kFThreads) void flex_lastq_kernel(FlexK a) {
     }
   }
   if (PASS == 2) {
-    // combine the chunk partials of each row in a fixed order
-    if (tid < bs) {
-      const float* pp = a.part + ((int64_t)h * a.nchunk) * bs * 2;
-      float mx = -INFINITY;
-      for (int c = 0; c < a.nchunk; ++c) mx = fmaxf(mx, pp[((int64_t)c * bs + tid) * 2]);
-      float s = 0.f;
-      for (int c = 0; c < a.nchunk; ++c) {
-        const float mc = pp[((int64_t)c * bs + tid) * 2], lc = pp[((int64_t)c * bs + tid) * 2 + 1];
-        if (mc > -INFINITY) s += lc * fexp2(mc - mx);
-      }
-      rowstat[tid * 2] = mx;
-      rowstat[tid * 2 + 1] = 1.0f / s;
+    // combine the chunk partials of each row in a fixed order: neighbouring
+    // lanes take every TPR-th chunk of a row, then a butterfly
+    constexpr int TPR = kFThreads / bs;
+    const int cr = tid / TPR, sub = tid % TPR;
+    const float2* pp = reinterpret_cast<const float2*>(a.part) + (int64_t)h * a.nchunk * bs + cr;
+    float mx = -INFINITY;
+#pragma unroll 4
+    for (int c = sub; c < a.nchunk; c += TPR) mx = fmaxf(mx, pp[(int64_t)c * bs].x);
+    for (int o = TPR / 2; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    float s = 0.f;
+#pragma unroll 4
+    for (int c = sub; c < a.nchunk; c += TPR) {
+      const float2 p = pp[(int64_t)c * bs];
+      s += p.x > -INFINITY ? p.y * fexp2(p.x - mx) : 0.f;
+    }
+    for (int o = TPR / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (sub == 0) {
+      rowstat[cr * 2] = mx;
+      rowstat[cr * 2 + 1] = 1.0f / s;
     }
     for (int e = tid; e < kFTile + bs; e += kFThreads) carry[e] = 0.f;
     __syncthreads();
@@ -344,18 +352,58 @@ __global__ __launch_bounds__(kFThreads) void flex_lastq_kernel(FlexK a) {
   }
 }
 
-// block means of K over each block's real rows (triton_bnhd_pool "avg", Flexprefill.py:656-782)
-template <typename T>
+// block means of K over each block's real rows (triton_bnhd_pool "avg", Flexprefill.py:656-782).  One
+// workgroup per 128 tokens of a KV head (128 / BS blocks): thread t loads 16 bytes (8 dims) of tokens
+// t / 16 + 16 u, all in flight together, adds its rows of each block, then the wave's four row groups and the
+// four waves in order (bound by the read of K; 32768 tokens of 8 heads at 32-token blocks 31.8 -> 12.8 us
+// against one thread per dim adding 2-byte loads row by row).
+constexpr int kPoolTok = 128;
+template <typename T, int BS>
 __global__ __launch_bounds__(kFThreads) void flex_kpool_kernel(const uint16_t* __restrict__ k, int64_t k_sh,
-                                                               int64_t k_sl, int L, int bs, int nb,
+                                                               int64_t k_sl, int L, int nb,
                                                                uint16_t* __restrict__ avg_k) {
-  const int hk = blockIdx.x / nb, j = blockIdx.x % nb;
-  const int t0 = j * bs, rows = min(bs, L - t0);
-  const uint16_t* src = k + (int64_t)hk * k_sh;
-  for (int d = threadIdx.x; d < kFD; d += kFThreads) {
-    float s = 0.f;
-    for (int r = 0; r < rows; ++r) s += to_f32(T{src[(int64_t)(t0 + r) * k_sl + d]});
-    avg_k[((int64_t)hk * nb + j) * kFD + d] = __builtin_bit_cast(uint16_t, Conv<T>::store(s / (float)rows));
+  constexpr int NB = kPoolTok / BS, U = kPoolTok / 16, UB = U / NB;   // blocks; rows per thread, per block
+  __shared__ float red[4][NB][kFD];
+  const int ng = (nb + NB - 1) / NB;
+  const int hk = blockIdx.x / ng, j0 = (blockIdx.x % ng) * NB;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = tid & 15;
+  const uint16_t* src = k + (int64_t)hk * k_sh + c * 8;
+  const int t0 = j0 * BS + (tid >> 4);
+  uint4 x[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) x[u] = *reinterpret_cast<const uint4*>(src + (int64_t)min(t0 + 16 * u, L - 1) * k_sl);
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    float s[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s[e] = 0.f;
+#pragma unroll
+    for (int v = 0; v < UB; ++v) {
+      const int u = b * UB + v;
+      const uint32_t w[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
+      const bool in = t0 + 16 * u < L;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float y = to_f32(T{(uint16_t)(w[e >> 1] >> (16 * (e & 1)))});
+        s[e] += in ? y : 0.f;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      s[e] += __shfl_xor(s[e], 16, 64);
+      s[e] += __shfl_xor(s[e], 32, 64);
+    }
+    if (lane < 16) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) red[wave][b][c * 8 + e] = s[e];
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < NB * kFD; i += kFThreads) {
+    const int b = i / kFD, d = i % kFD, j = j0 + b;
+    if (j >= nb) break;
+    const float s = ((red[0][b][d] + red[1][b][d]) + red[2][b][d]) + red[3][b][d];
+    avg_k[((int64_t)hk * nb + j) * kFD + d] = __builtin_bit_cast(uint16_t, Conv<T>::store(s / (float)min(BS, L - j * BS)));
   }
 }
 
@@ -1158,9 +1206,20 @@ struct FlexLayout {
 
 // sparse: whether any head can take the block-level cover (tau > 0; the
 // square-root JS divergence is >= 0, or nan, so js < tau never holds otherwise)
+// Key columns per workgroup of the last-block passes: halved while the heads'
+// chunks leave workgroup slots empty (a chunk is a serial chain of 128-key
+// tiles), down to 512, where the second pass's extra tile per chunk costs a
+// fourth.  Both passes, 32 heads, 2048 against this: 8192 tokens 32-token blocks
+// 92 -> 47 us, 128-token blocks 262 -> 111; 32768 tokens 124 -> 121.
+static int flex_chunk(int Hq, int L) {
+  int c = kFChunk;
+  while (c > kFChunkMin && (int64_t)Hq * ((L + c - 1) / c) < 1024) c >>= 1;
+  return c;
+}
+
 static FlexLayout flex_work(int Hq, int Hk, int L, int bs, bool sparse) {
   const int nb = (L + bs - 1) / bs;
-  const int nchunk = (L + kFChunk - 1) / kFChunk;
+  const int chunk = flex_chunk(Hq, L), nchunk = (L + chunk - 1) / chunk;
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t at = off;
@@ -1206,7 +1265,7 @@ static void launch_cut_passes(const CutJobs& c, hipStream_t s) {
 template <typename T>
 static int launch_flex(const fs_flex_args& a, hipStream_t s) {
   const int nb = (a.L + a.bs - 1) / a.bs;
-  const int nchunk = (a.L + kFChunk - 1) / kFChunk;
+  const int chunk = flex_chunk(a.Hq, a.L), nchunk = (a.L + chunk - 1) / chunk;
   const bool sparse = a.tau > 0.f;
   const FlexLayout lay = flex_work(a.Hq, a.Hk, a.L, a.bs, sparse);
   char* w = static_cast<char*>(a.work);
@@ -1216,6 +1275,7 @@ static int launch_flex(const fs_flex_args& a, hipStream_t s) {
   k.q_sh = a.q_sh; k.q_sl = a.q_sl; k.k_sh = a.k_sh; k.k_sl = a.k_sl;
   k.Hq = a.Hq; k.Hk = a.Hk; k.L = a.L; k.bs = a.bs; k.nb = nb; k.gqa_interleave = a.gqa_interleave;
   k.nchunk = nchunk;
+  k.chunk = chunk;
   k.sqrt_d = (float)sqrt((double)a.D);
   k.part = reinterpret_cast<float*>(w + lay.part);
   k.vert = a.vertical ? a.vertical : reinterpret_cast<float*>(w + lay.vert);
@@ -1233,7 +1293,10 @@ static int launch_flex(const fs_flex_args& a, hipStream_t s) {
                             : launch_lastq<T, 128>(k, grid, smem1, smem2, s))
     return rc;
   uint16_t* avg_k = reinterpret_cast<uint16_t*>(w + lay.avgk);
-  flex_kpool_kernel<T><<<(unsigned)(a.Hk * nb), kFThreads, 0, s>>>(k.k, a.k_sh, a.k_sl, a.L, a.bs, nb, avg_k);
+  const unsigned pgrid = (unsigned)(a.Hk * ((a.L + kPoolTok - 1) / kPoolTok));
+  auto kpool = a.bs == 16 ? flex_kpool_kernel<T, 16> : a.bs == 32 ? flex_kpool_kernel<T, 32>
+               : a.bs == 64 ? flex_kpool_kernel<T, 64> : flex_kpool_kernel<T, 128>;
+  kpool<<<pgrid, kFThreads, 0, s>>>(k.k, a.k_sh, a.k_sl, a.L, nb, avg_k);
   if (int rc = fs_host::launch_status("fs_flex (scores)")) return rc;
   // the profiles' mass cuts at gamma (each profile adds to one: masses x 2^58)
   CutJobs pc{};
