@@ -125,6 +125,10 @@ __device__ __forceinline__ void score_panel(const T* qb, const T* kb, int D, int
 #pragma unroll
         for (int st = 0; st < kSteps; ++st) kv[u][st] = row_chunk<T, WIDE>(krow, d0 + (4 * st + g) * V, D, true);
       }
+      // the query chunks are whole before the chains start: selected between the
+      // MFMAs, they made the register allocator move an accumulator mid-chain
+#pragma unroll
+      for (int st = 0; st < kSteps; ++st) asm volatile("" : "+v"(qv[st].x), "+v"(qv[st].y), "+v"(qv[st].z), "+v"(qv[st].w));
 #pragma unroll
       for (int st = 0; st < kSteps; ++st)
 #pragma unroll
