@@ -26,8 +26,8 @@
 //    wait overlaps the other's MFMAs).
 //  - BS = 64 uses TK = 64 split between two key groups (4 waves), merged
 //    through LDS at the end.
-//  - 16- and 32-token block lists run in union mode: a workgroup of 128
-//    queries walks the union of its 128 / bs rows' lists (see below), with the
+//  - 16- and 32-token block lists run in union mode: a workgroup of 64 or 128
+//    queries walks the union of its rows' lists (see below), with the BS = 64 or
 //    BS = 128 layout.  Dense calls at those block sizes take the BS = 128 kernel.
 // LDS rows are 256 B with the 16-byte chunk c of row r stored at c ^ (r & 15)
 // so the 8 lanes of a ds_read_b128 phase hit distinct banks.
@@ -238,13 +238,14 @@ __device__ __forceinline__ uint4 lds16(const char* base, uint32_t off) {
   return *reinterpret_cast<const uint4*>(base + off);
 }
 
-// LB < BS (union mode, BS = 128): the block lists are at LB-token granularity
-// and a workgroup covers BS / LB consecutive list rows (128 queries).  It walks
-// the ascending union of their lists (union_kernel), each entry a key block
-// with the set of the group's rows that selected it; a lane's scores of a key
-// block its row did not select are masked.  A tile of TK keys holds TK / LB
-// union entries, so every K / V^T tile copy serves 128 queries and every wave
-// does 32 x TK per barrier, as with 128-token blocks.
+// LB < BS (union mode): the block lists are at LB-token granularity and a
+// workgroup covers BS / LB consecutive list rows (BS = 64 or 128 queries, see
+// union_queries).  It walks the ascending union of their lists (union_kernel),
+// each entry a key block with the set of the group's rows that selected it; a
+// lane's scores of a key block its row did not select are masked.  A tile of TK
+// keys holds TK / LB union entries, so every K / V^T tile copy serves BS queries
+// and a wave works at the rate it has with BS-token blocks.  At BS = 64 and
+// LB = 32 each wave's share of a tile is one list row and one entry.
 //
 // VD (V direct): no V^T pre-pass.  V tiles are copied as they are, [TK][D], and
 // each operand of P V is two transposing LDS reads (ds_read_b64_tr_b16) instead
@@ -266,7 +267,7 @@ void bsattn_kernel(AttnKArgs a) {
   constexpr bool UNION = LB < BS;
   constexpr int EPT = UNION ? TK / LB : 1;         // union entries per tile
   static_assert(!(UNION && VD), "union mode reads V^T");
-  static_assert(!UNION || (BS == 128 && TK == 64 && (LB == 16 || LB == 32)), "union mode: 16- or 32-token lists");
+  static_assert(!UNION || (TK == 64 && (LB == 16 || LB == 32)), "union mode: 16- or 32-token lists");
   using Ops = MfmaOps<T>;
   using V8 = typename Ops::V8;
   // [K | V^T][buffer] tiles; 256-byte rows with swizzled 16-byte chunks
@@ -649,18 +650,20 @@ void bsattn_kernel(AttnKArgs a) {
   auto mask_only = [&](int key0, f32x16_t* s, TileEnt ue) {
     if constexpr (UNION) {
       if (listed) {
-        // key0 is the tile index.  Lane row jq of the group; a key of entry ie
-        // is kept iff the entry is real, row jq selected it, and it is below Lk
-        // and (causal) at or before the lane's query.  Fast path: every row of
-        // this wave selected every entry and no key needs the causal / Lk cut.
+        // key0 is the tile index.  Lane row jq of the group; a key of one of
+        // this wave's EPW entries is kept iff the entry is real, row jq selected
+        // it, and it is below Lk and (causal) at or before the lane's query.
+        // Fast path: every row of this wave selected every entry of it and no
+        // key needs the causal / Lk cut.
         const int jq = (qq * 32 + l32) / LB;
         constexpr uint32_t kWaveRows = (1u << (32 / LB)) - 1;
         const uint32_t wrows = kWaveRows << ((qq * 32) / LB);
-        uint32_t ents[EPT];
+        constexpr int EPW = C::KH / LB;            // entries of this wave's key group
+        uint32_t ents[EPW];
         bool full = true;
 #pragma unroll
-        for (int ie = 0; ie < EPT; ++ie) {
-          ents[ie] = ue.e[ie];
+        for (int ie = 0; ie < EPW; ++ie) {
+          ents[ie] = C::KG == 2 && kh ? ue.e[EPT - EPW + ie] : ue.e[ie];
           const int blk = (int)(ents[ie] & 0xffffu);
           if (blk >= a.Nk || ((ents[ie] >> 16) & wrows) != wrows || blk * LB + LB > a.Lk ||
               (a.is_causal && blk * LB + LB - 1 > qw0 + off))
@@ -668,7 +671,7 @@ void bsattn_kernel(AttnKArgs a) {
         }
         if (!full) {
 #pragma unroll
-          for (int ie = 0; ie < EPT; ++ie) {
+          for (int ie = 0; ie < EPW; ++ie) {
             const int blk = (int)(ents[ie] & 0xffffu);
             const bool mine = blk < a.Nk && ((ents[ie] >> (16 + jq)) & 1u);
             int lim = a.Lk - blk * LB;
@@ -972,6 +975,8 @@ constexpr int kPoolPercent = 10;                 // share of the work units (the
 constexpr int kOrderMaxBins = 8192;
 constexpr int64_t kDirectMaxKeys = 49152;        // see v_direct
 constexpr int64_t kDirectMaxKeysDense = 24576;
+constexpr int kUnion64MaxKeys = 40960;           // see union_queries
+constexpr int kUnion64MaxKeys16 = 32768;
 constexpr int kOrderKeysPerThread = 8;           // keys kept in registers between the two passes
 // kvmajor = 0: one longest-first order over all units (the KV group left out of the key).
 __global__ __launch_bounds__(kOrderThreads) void order_kernel(const int32_t* __restrict__ cnt, int Hq, int Hk,
@@ -1203,9 +1208,26 @@ static bool dense_by_64(const fs_attn_args& a, int Nq128) {
   const int64_t wg = (int64_t)a.B * a.Hq * Nq128;
   return wg <= 384 || (wg <= 512 && a.Lk >= 960);
 }
+// Queries of a workgroup in union mode.  A group of 64 has fewer entries that
+// some of its rows did not select (FlexPrefill's lists of 32768 tokens, gamma
+// 0.95: the rows select 76% of a union over 128 queries and 88% of one over 64
+// at 32-token blocks, 42% and 58% at 16) and gives a short call twice the workgroups,
+// but a tile copy serves half as many queries, and past the last-level cache the
+// copies bound the loop.  Whole FlexPrefill calls (gamma 0.95), 128 against 64:
+//   block 32, 32 / 8 heads: 4100 tokens 376 / 358 us, 9001 796 / 734, 32768 8010 /
+//     7705 (tau 0: 6238 / 5366), 65536 29.65 / 30.39 ms, 98304 63.8 / 64.8;
+//     32 / 32 heads: 40000 11120 / 10775 us; 16 / 2: 16000 1068 / 1025;
+//   block 16: 9000 (tau 0) 672 / 618, 30000 7172 / 7077.
+// Lists that select nearly everything lose: random masks of 16384 tokens, block
+// 32, at density 0.1 / 0.5 / 1 take 928 / 2328 / 2375 us by 128 and 747 / 2255 / 2633
+// by 64.  The lists are on the device, so the line is at the length alone.  At
+// D = 64 groups of 128 stay: 645 / 1592 / 1403 against 540 / 1651 / 1748.
+static int union_queries(const fs_attn_args& a) {
+  return a.D == 128 && a.Lk <= (a.bs == 32 ? kUnion64MaxKeys : kUnion64MaxKeys16) ? 64 : 128;
+}
 static int union_groups(const fs_attn_args& a) {
   const int Nq = (a.Lq + a.bs - 1) / a.bs;
-  const int R = 128 / a.bs;
+  const int R = union_queries(a) / a.bs;
   return (Nq + R - 1) / R;
 }
 
@@ -1261,10 +1283,10 @@ static int launch_run(const fs_attn_args& a, int Nq, int Nk, hipStream_t s, int 
 }
 
 // union mode (16- and 32-token lists): union lists, order pass over the
-// groups, the 128-query kernel over the unions
-template <int LB, typename T, int D>
+// groups of Q queries, the kernel over the unions
+template <int Q, int LB, typename T, int D>
 static int launch_run_union(const fs_attn_args& a, hipStream_t s) {
-  constexpr int R = 128 / LB;
+  constexpr int R = Q / LB;
   const int NqL = (a.Lq + LB - 1) / LB, NkL = (a.Lk + LB - 1) / LB;
   const int Ng = (NqL + R - 1) / R;
   char* w = static_cast<char*>(a.work);
@@ -1301,7 +1323,7 @@ static int launch_run_union(const fs_attn_args& a, hipStream_t s) {
   k.ctr = ctr;
   k.gqa_interleave = a.gqa_interleave ? 1 : 0;
   const unsigned grid = deal_units(total, run, k.static_units, k.pool_units);
-  bsattn_kernel<128, 64, T, LB, D><<<grid, AttnCfg<128, 64, D>::NT, 0, s>>>(k);
+  bsattn_kernel<Q, 64, T, LB, D><<<grid, AttnCfg<Q, 64, D>::NT, 0, s>>>(k);
   return fs_host::launch_status("fs_bsattn");
 }
 
@@ -1380,8 +1402,13 @@ static int run_typed(const fs_attn_args* a, int Nq, int Nk, hipStream_t s) {
 }
 template <typename T, int D>
 static int run_head(const fs_attn_args* a, int Nq, int Nk, hipStream_t s) {
-  // 16- and 32-token lists: unions over groups of 128 queries
-  if (union_mode(*a)) return a->bs == 32 ? launch_run_union<32, T, D>(*a, s) : launch_run_union<16, T, D>(*a, s);
+  // 16- and 32-token lists: unions over groups of 64 or 128 queries
+  if (union_mode(*a)) {
+    if constexpr (D == 128) {
+      if (union_queries(*a) == 64) return a->bs == 32 ? launch_run_union<64, 32, T, D>(*a, s) : launch_run_union<64, 16, T, D>(*a, s);
+    }
+    return a->bs == 32 ? launch_run_union<128, 32, T, D>(*a, s) : launch_run_union<128, 16, T, D>(*a, s);
+  }
   return v_direct(*a) ? run_typed<T, D, true>(a, Nq, Nk, s) : run_typed<T, D, false>(a, Nq, Nk, s);
 }
 

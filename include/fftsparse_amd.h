@@ -345,8 +345,8 @@ FS_API int fs_flex(const fs_flex_args* a, void* stream);
  * blk_cnt == NULL selects every key block up to the
  * causal limit (dense causal attention).  Supported: dtype bf16/f16, D in {64, 128},
  * bs in {16, 32, 64, 128} (16 and 32: FlexPrefill's block sizes; their masks
- * are attended 128 queries at a time over the union of 128 / bs rows,
- * up to 8192 key blocks).  All tensors are
+ * are attended 64 or 128 queries at a time (64 at D = 128 up to 40960 keys,
+ * 32768 at bs = 16) over the union of those rows' lists, up to 8192 key blocks).  All tensors are
  * strided views with d contiguous.
  * work: fs_bsattn_work_bytes(a) bytes of device scratch (V may be staged there
  * transposed, and the work items' longest-first order and the counters from

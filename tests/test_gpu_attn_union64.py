@@ -1,0 +1,58 @@
+"""Attention over 16- and 32-token block lists in groups of 64 and of 128 queries:
+lengths at the edges of a group, entries selected by one row of a group only,
+rows that select nothing, and the length at which the group size changes."""
+import pytest
+import torch
+
+import fftsparse_amd
+from fftsparse_amd.attn import bits_from_mask
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(q, k, v, mask, bs, rows):
+    """fp32 attention of the given query rows; a row that selects no key is 0."""
+    G = q.shape[1] // k.shape[1]
+    L, D = q.shape[2:]
+    kf, vf = k[0].float().repeat_interleave(G, 0), v[0].float().repeat_interleave(G, 0)
+    s = torch.stack([q[0, h, rows].float() @ kf[h].T.contiguous() for h in range(q.shape[1])]) / D ** 0.5
+    j = torch.arange(L, device=q.device)
+    keep = mask[:, rows // bs][:, :, j // bs] & (j[None] <= rows[:, None])[None]
+    p = torch.nan_to_num(torch.softmax(s.masked_fill(~keep, float("-inf")), -1))
+    return torch.stack([p[h] @ vf[h] for h in range(q.shape[1])])
+
+
+@pytest.mark.parametrize("L,bs,D,density,dtype", [
+    (64, 32, 128, 0.6, torch.bfloat16),           # one group
+    (65, 16, 128, 0.6, torch.float16),            # one row past a group
+    (127, 16, 64, 0.5, torch.bfloat16),           # head dim 64: groups of 128
+    (129, 16, 128, 0.5, torch.bfloat16),
+    (700, 32, 128, 0.05, torch.float16),          # entries of one row, empty rows
+    (1999, 16, 128, 0.02, torch.bfloat16),
+    (1025, 32, 128, 1.0, torch.bfloat16),
+    (40960, 32, 128, 0.02, torch.bfloat16),       # the last length in groups of 64
+    (40961, 32, 128, 0.02, torch.bfloat16),       # the first in groups of 128
+    (32769, 16, 128, 0.01, torch.bfloat16),       # likewise at 16-token blocks
+])
+def test_union_groups(L, bs, D, density, dtype):
+    print(f"[case] union groups L={L} bs={bs} D={D} density={density} {dtype}", flush=True)
+    Hq, Hk = 4, 2
+    g = torch.Generator(device="cuda").manual_seed(L + bs)
+    q, k, v = (torch.randn(1, h, L, D, generator=g, device="cuda").to(dtype) for h in (Hq, Hk, Hk))
+    N = -(-L // bs)
+    mask = torch.rand(Hq, N, N, generator=g, device="cuda") < density
+    mask[:, 1::5] = False                          # rows that select nothing
+    cnt, bits = bits_from_mask(mask)
+    out = fftsparse_amd.block_sparse_attention(q, k, v, cnt, bits, block_size=bs)
+    out = out.view(L, Hq, D).transpose(0, 1).float()
+    rows = torch.arange(L, device="cuda")
+    if L > 4096:
+        rows = torch.cat([rows[:130], rows[::613], rows[-130:]])
+    ref = reference(q, k, v, mask, bs, rows)
+    got = out[:, rows]
+    # P and the output are rounded to the 16-bit type: each entry of P to 2^-9 (bf16)
+    # of itself, so a row errs by 2^-9 max |V| (about 5) at most, and its store by 2^-9 |out|
+    eps = 2.0 ** (-9 if dtype == torch.bfloat16 else -12)
+    assert (got - ref).abs().max().item() <= 2 * eps * v.float().abs().max().item()
+    empty = ~mask.any(-1)[:, rows // bs]
+    assert (got[empty] == 0).all()
