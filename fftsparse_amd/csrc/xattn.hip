@@ -425,7 +425,12 @@ void xattn_scores_wide_kernel(XScoreK a) {
   }
 }
 
-// pass 2 over the stored scores
+// pass 2 over the stored scores.  A workgroup walks its rows in order; the
+// loads of kXSumRows rows are issued together, and only the keys at a row's end
+// are tested one by one.  Bound by the exponentials' VALU work: 32768 tokens, 32
+// heads, stride 8: 232 us one row at a time with every key tested, 213 with the
+// loads together, 161 now (3.3 TB/s of scores).
+constexpr int kXSumRows = 8;
 template <typename T, bool TP>
 __global__ __launch_bounds__(kXThreads) void xattn_sums_kernel(XScoreK a) {
   __shared__ float rm[kXRows], rl[kXRows];
@@ -482,34 +487,54 @@ __global__ __launch_bounds__(kXThreads) void xattn_sums_kernel(XScoreK a) {
     const int n = c0 + 8 * tid;
     const bool key_in = n < NK;                      // NK and n are multiples of 8
     float acc = 0.f;
-    for (int i = 0; i < nr; ++i) {
-      const int row = r0 + i;
-      float v = 0.f;
-      // a row's visible keys start and end on multiples of 8 from below (chunk
-      // starts are multiples of bs / S >= 8), so n decides whether any is seen
-      if (key_in && rok[i] && xkey_ok<TP>(a, row, n)) {
-        const uint4 w = *reinterpret_cast<const uint4*>(src + (int64_t)i * NK + n);
-        const uint32_t pr[4] = {w.x, w.y, w.z, w.w};
+    uint4 w[kXSumRows];
+    bool seen[kXSumRows];
+    for (int i0 = 0; i0 < nr; i0 += kXSumRows) {
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          const uint16_t e = (uint16_t)((t & 1) ? (pr[t >> 1] >> 16) : (pr[t >> 1] & 0xffffu));
-          if (xkey_ok<TP>(a, row, n + t)) v += prob(i, xscaled<T, TP>(a, to_f32(T{e})));
+      for (int u = 0; u < kXSumRows; ++u) {
+        // a row's visible keys start and end on multiples of 8 from below (chunk
+        // starts are multiples of bs / S >= 8), so n decides whether any is seen
+        const int i = i0 + u;
+        seen[u] = i < nr && key_in && rok[i] && xkey_ok<TP>(a, r0 + i, n);
+        w[u] = seen[u] ? *reinterpret_cast<const uint4*>(src + (int64_t)i * NK + n) : make_uint4(0, 0, 0, 0);
+      }
+#pragma unroll
+      for (int u = 0; u < kXSumRows; ++u) {
+        const int i = i0 + u, row = r0 + i;
+        if (i >= nr) break;
+        float v = 0.f;
+        if (seen[u]) {
+          const uint32_t pr[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+          // the first of the 8 keys is seen: with the last one all are
+          const bool all = xkey_ok<TP>(a, row, n + 7);
+          float p[8];
+#pragma unroll
+          for (int t = 0; t < 8; ++t) {
+            const uint16_t e = (uint16_t)((t & 1) ? (pr[t >> 1] >> 16) : (pr[t >> 1] & 0xffffu));
+            p[t] = prob(i, xscaled<T, TP>(a, to_f32(T{e})));
+          }
+          if (!all) {
+#pragma unroll
+            for (int t = 1; t < 8; ++t) p[t] = xkey_ok<TP>(a, row, n + t) ? p[t] : 0.f;
+          }
+#pragma unroll
+          for (int t = 0; t < 8; ++t) v += p[t];
         }
-      }
-      if constexpr (TP) {
-        // the row's sum over the block's keys, rounded to dtype
-        for (int o = 1; o < gl; o <<= 1) v += __shfl_xor(v, o, 64);
-        acc += Conv<T>::round(v);
-      } else {
-        acc += v;
-      }
-      if ((i + 1) % rpb == 0) {                      // the end of a block row
-        float tot = acc;
-        if constexpr (!TP) for (int o = 1; o < gl; o <<= 1) tot += __shfl_xor(tot, o, 64);
-        const int I = row / rpb, J = n / rbs;
-        if (key_in && (tid % gl) == 0 && I < a.Nb && J < a.Nb && (!a.causal || J <= I))
-          a.sums[((int64_t)h * a.Nb + I) * a.Nb + J] = Conv<T>::round(tot);
-        acc = 0.f;
+        if constexpr (TP) {
+          // the row's sum over the block's keys, rounded to dtype
+          for (int o = 1; o < gl; o <<= 1) v += __shfl_xor(v, o, 64);
+          acc += Conv<T>::round(v);
+        } else {
+          acc += v;
+        }
+        if ((i + 1) % rpb == 0) {                      // the end of a block row
+          float tot = acc;
+          if constexpr (!TP) for (int o = 1; o < gl; o <<= 1) tot += __shfl_xor(tot, o, 64);
+          const int I = row / rpb, J = n / rbs;
+          if (key_in && (tid % gl) == 0 && I < a.Nb && J < a.Nb && (!a.causal || J <= I))
+            a.sums[((int64_t)h * a.Nb + I) * a.Nb + J] = Conv<T>::round(tot);
+          acc = 0.f;
+        }
       }
     }
   }
