@@ -367,8 +367,9 @@ class AttentionCall:
     """One prepared stage-2 call: argument struct, workspace and output.
 
     ``prepare()`` stages V^T in the workspace (fs_bsattn_prepare), ``run()``
-    orders the work items and runs the attention kernel (fs_bsattn_run), and
-    ``__call__`` does both in one C call (fs_bsattn).  Every launch goes on
+    orders the work items and runs the attention kernel (fs_bsattn_run) on V as
+    ``prepare()`` found it, and ``__call__`` does both in one C call (fs_bsattn),
+    which reads V in place where it is used few times.  Every launch goes on
     torch's current stream."""
 
     def __init__(self, query_states, key_states, value_states, blk_cnt=None, blk_bits=None, *,

@@ -2,8 +2,8 @@
 // Role: block_sparse_attn_func (my_attn_v7.py:775-786) and, with no block
 // list, flash_attn_func(causal=True) (my_attn_v7.py:509-519).
 //
-// Pre-pass (vt_kernel; not where v_direct holds, see VD): V [Lk][D] of every KV
-// head is rewritten once per call as V^T [D][Lp] (Lp = Nk * BS rounded up to 64, zero padded) with the keys of every group of
+// Pre-pass (vt_kernel; left out of a whole call where v_direct holds, see VD): V
+// [Lk][D] of every KV head is rewritten once per call as V^T [D][Lp] (Lp = Nk * BS rounded up to 64, zero padded) with the keys of every group of
 // 16 stored in the order 0-3, 8-11, 4-7, 12-15.  With 16- or 32-token block
 // lists (union mode) V^T is stored block by block instead, [Lp / bs][D][bs]:
 // the copy of one listed block is then one contiguous run of D * bs keys
@@ -1155,8 +1155,8 @@ static int kv_major(const fs_attn_args& a, int Nq) {
   return per_group >= 4 * 2 * (int64_t)n ? 1 : 0;
 }
 
-// V is read as it is (no V^T pre-pass) where V is used few times: the pre-pass
-// moves V twice and is a launch (6 us at 1000 tokens, 26 us at 8192 with 32 KV
+// fs_bsattn reads V as it is (no V^T pre-pass) where V is used few times: the
+// pre-pass moves V twice and is a launch (6 us at 1000 tokens, 26 us at 8192 with 32 KV
 // heads), the direct loop takes 1-3% longer, so the line is at a count of query
 // heads per KV head x keys.  Whole calls, V^T against direct, bf16, D = 128:
 //   dense  1000 tokens, 32 / 8 heads (4000): 29.5 / 23.6 us; 4096 (16384): 164 / 158;
@@ -1170,8 +1170,9 @@ static bool v_direct(const fs_attn_args& a) {
   return (int64_t)(a.Hq / a.Hk) * a.Lk <= (a.blk_cnt != nullptr ? kDirectMaxKeys : kDirectMaxKeysDense);
 }
 
+// Every workspace has room for V^T, whatever v_direct says: fs_bsattn_prepare
+// stages it for any fs_bsattn_run that shares v, Lk, bs and lists (present or not).
 static size_t vt_bytes(const fs_attn_args& a) {
-  if (v_direct(a)) return 0;
   const int Nk = (a.Lk + a.bs - 1) / a.bs;
   return ((size_t)a.B * a.Hk * a.D * vt_len(Nk, a.bs) * 2 + 255) & ~(size_t)255;
 }
@@ -1333,7 +1334,7 @@ using namespace fs;
 
 extern "C" size_t fs_bsattn_work_bytes(const fs_attn_args* a) {
   if (!a || a->B <= 0 || a->Hq <= 0 || a->Hk <= 0 || a->Lq <= 0 || a->Lk <= 0 || a->D <= 0 || a->bs <= 0) return 0;
-  size_t n = vt_bytes(*a) + order_bytes(*a);       // never 0
+  size_t n = vt_bytes(*a) + order_bytes(*a);
   if (union_mode(*a)) {
     const size_t Ng = (size_t)union_groups(*a), Nk = (size_t)(a->Lk + a->bs - 1) / a->bs;
     n += align256((size_t)a->Hq * Ng * sizeof(int32_t)) + (size_t)a->Hq * Ng * Nk * sizeof(uint32_t);
@@ -1379,7 +1380,6 @@ static int check_attn(const fs_attn_args* a, const char* fn) {
 
 extern "C" int fs_bsattn_prepare(const fs_attn_args* a, void* stream) {
   if (int rc = check_attn(a, "fs_bsattn_prepare")) return rc;
-  if (v_direct(*a)) return FS_OK;                  // V is read as it is
   const int Nk = (a->Lk + a->bs - 1) / a->bs;
   const int Lp = vt_len(Nk, a->bs);
   auto vt = a->D == 64 ? vt_kernel<64> : vt_kernel<128>;
@@ -1401,7 +1401,7 @@ static int run_typed(const fs_attn_args* a, int Nq, int Nk, hipStream_t s) {
   return launch_run<128, 64, T, D, VD>(*a, Nq128, Nk128, s, Lp);
 }
 template <typename T, int D>
-static int run_head(const fs_attn_args* a, int Nq, int Nk, hipStream_t s) {
+static int run_head(const fs_attn_args* a, int Nq, int Nk, bool direct, hipStream_t s) {
   // 16- and 32-token lists: unions over groups of 64 or 128 queries
   if (union_mode(*a)) {
     if constexpr (D == 128) {
@@ -1409,21 +1409,28 @@ static int run_head(const fs_attn_args* a, int Nq, int Nk, hipStream_t s) {
     }
     return a->bs == 32 ? launch_run_union<128, 32, T, D>(*a, s) : launch_run_union<128, 16, T, D>(*a, s);
   }
-  return v_direct(*a) ? run_typed<T, D, true>(a, Nq, Nk, s) : run_typed<T, D, false>(a, Nq, Nk, s);
+  return direct ? run_typed<T, D, true>(a, Nq, Nk, s) : run_typed<T, D, false>(a, Nq, Nk, s);
+}
+
+// the kernels after the pre-pass; direct: V is read as it is (checked arguments)
+static int run_attn(const fs_attn_args* a, bool direct, hipStream_t s) {
+  const int Nq = (a->Lq + a->bs - 1) / a->bs;
+  const int Nk = (a->Lk + a->bs - 1) / a->bs;
+  if (a->D == 64)
+    return a->dtype == FS_DTYPE_BF16 ? run_head<bf16_t, 64>(a, Nq, Nk, direct, s)
+                                     : run_head<f16_t, 64>(a, Nq, Nk, direct, s);
+  return a->dtype == FS_DTYPE_BF16 ? run_head<bf16_t, 128>(a, Nq, Nk, direct, s)
+                                   : run_head<f16_t, 128>(a, Nq, Nk, direct, s);
 }
 
 extern "C" int fs_bsattn_run(const fs_attn_args* a, void* stream) {
   if (int rc = check_attn(a, "fs_bsattn_run")) return rc;
-  const int Nq = (a->Lq + a->bs - 1) / a->bs;
-  const int Nk = (a->Lk + a->bs - 1) / a->bs;
-  hipStream_t s = (hipStream_t)stream;
-  if (a->D == 64)
-    return a->dtype == FS_DTYPE_BF16 ? run_head<bf16_t, 64>(a, Nq, Nk, s) : run_head<f16_t, 64>(a, Nq, Nk, s);
-  return a->dtype == FS_DTYPE_BF16 ? run_head<bf16_t, 128>(a, Nq, Nk, s) : run_head<f16_t, 128>(a, Nq, Nk, s);
+  return run_attn(a, false, (hipStream_t)stream);
 }
 
 extern "C" int fs_bsattn(const fs_attn_args* a, void* stream) {
   if (int rc = check_attn(a, "fs_bsattn")) return rc;
+  if (v_direct(*a)) return run_attn(a, true, (hipStream_t)stream);
   if (int rc = fs_bsattn_prepare(a, stream)) return rc;
-  return fs_bsattn_run(a, stream);
+  return run_attn(a, false, (hipStream_t)stream);
 }

@@ -1,0 +1,50 @@
+"""What a caller of the attention may rely on besides its result: the two halves
+of the call (prepare stages V, run reads what was staged)."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from fftsparse_amd import AttentionCall, block_sparse_attention
+from fftsparse_amd.attn import bits_from_mask
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+def _qkv(L, Hq, Hk, D=128, dtype=torch.bfloat16, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(1, h, L, D, generator=g).to(dtype).to(DEV) for h in (Hq, Hk, Hk)]
+
+
+def _lists(Hq, L, bs, density, seed=0):
+    n = -(-L // bs)
+    mask = torch.rand(Hq, n, n, generator=torch.Generator().manual_seed(seed)) < density
+    return [t.to(DEV) for t in bits_from_mask(mask)]
+
+
+@pytest.mark.parametrize("L,bs,listed", [(700, 128, False), (333, 32, False), (1500, 128, True), (1000, 64, True),
+                                         (900, 32, True)])
+def test_run_reads_v_as_it_was_prepared(L, bs, listed):
+    q, k, v = _qkv(L, 4, 2, seed=L)
+    lists = _lists(4, L, bs, 0.6) if listed else (None, None)
+    ref = block_sparse_attention(q, k, v, *lists, block_size=bs)
+    call = AttentionCall(q, k, v, *lists, block_size=bs)
+    call.prepare()
+    v.fill_(float("nan"))
+    assert torch.equal(call.run(), ref)
+
+
+@pytest.mark.parametrize("listed", [False, True])
+def test_prepare_serves_every_query_head_count(listed):
+    """2 and 64 query heads on the same 2 KV heads and workspace: few and many uses of V."""
+    L, Hk = 2100, 2
+    q, k, v = _qkv(L, 64, Hk, seed=3)
+    lists = [_lists(h, L, 128, 0.5) if listed else (None, None) for h in (Hk, 64)]
+    few = AttentionCall(q[:, :Hk], k, v, *lists[0])
+    many = AttentionCall(q, k, v, *lists[1])
+    ref = block_sparse_attention(q, k, v, *lists[1])
+    many.work.zero_()
+    few.args.work = many.args.work
+    few.prepare()
+    assert torch.equal(many.run(), ref)
