@@ -1155,6 +1155,22 @@ static int kv_major(const fs_attn_args& a, int Nq) {
   return per_group >= 4 * 2 * (int64_t)n ? 1 : 0;
 }
 
+// Whether the output's storage meets V's (the spans of the two views, so views
+// interleaved in one buffer count): out may replace v, whose rows other
+// workgroups still read when it is written.
+static bool out_meets_v(const fs_attn_args& a) {
+  auto span = [&](const void* p, const int64_t (&st)[3], const int (&n)[3], uintptr_t& lo, uintptr_t& hi) {
+    int64_t l = 0, h = a.D;
+    for (int i = 0; i < 3; ++i) (st[i] < 0 ? l : h) += st[i] * (n[i] - 1);
+    lo = (uintptr_t)p + (uintptr_t)(2 * l);
+    hi = (uintptr_t)p + (uintptr_t)(2 * h);
+  };
+  uintptr_t v0, v1, o0, o1;
+  span(a.v, {a.v_sb, a.v_sh, a.v_sl}, {a.B, a.Hk, a.Lk}, v0, v1);
+  span(a.out, {a.o_sb, a.o_sh, a.o_sl}, {a.B, a.Hq, a.Lq}, o0, o1);
+  return v0 < o1 && o0 < v1;
+}
+
 // fs_bsattn reads V as it is (no V^T pre-pass) where V is used few times: the
 // pre-pass moves V twice and is a launch (6 us at 1000 tokens, 26 us at 8192 with 32 KV
 // heads), the direct loop takes 1-3% longer, so the line is at a count of query
@@ -1430,7 +1446,7 @@ extern "C" int fs_bsattn_run(const fs_attn_args* a, void* stream) {
 
 extern "C" int fs_bsattn(const fs_attn_args* a, void* stream) {
   if (int rc = check_attn(a, "fs_bsattn")) return rc;
-  if (v_direct(*a)) return run_attn(a, true, (hipStream_t)stream);
+  if (v_direct(*a) && !out_meets_v(*a)) return run_attn(a, true, (hipStream_t)stream);
   if (int rc = fs_bsattn_prepare(a, stream)) return rc;
   return run_attn(a, false, (hipStream_t)stream);
 }

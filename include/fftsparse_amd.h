@@ -370,7 +370,7 @@ typedef struct {
 FS_API size_t fs_bsattn_work_bytes(const fs_attn_args* a);
 /* The whole stage-2 call: the result of fs_bsattn_prepare then fs_bsattn_run,
  * bit for bit.  Where V is used few times (a short sequence, few query heads per
- * KV head) it reads v as it is and stages nothing. */
+ * KV head, an out apart from v's storage) it reads v as it is and stages nothing. */
 FS_API int fs_bsattn(const fs_attn_args* a, void* stream);
 /* The two halves of fs_bsattn, for callers that time or reuse them apart.
  * prepare: writes V^T of every KV head into work (depends on v, and on bs

@@ -1,5 +1,6 @@
 """What a caller of the attention may rely on besides its result: the two halves
-of the call (prepare stages V, run reads what was staged)."""
+of the call (prepare stages V, run reads what was staged), and an output that
+takes V's place."""
 from __future__ import annotations
 
 import pytest
@@ -48,3 +49,18 @@ def test_prepare_serves_every_query_head_count(listed):
     few.args.work = many.args.work
     few.prepare()
     assert torch.equal(many.run(), ref)
+
+
+@pytest.mark.parametrize("L,bs,listed", [(700, 128, False), (2000, 128, False), (3000, 128, True), (2500, 64, True),
+                                         (1500, 32, True)])
+def test_output_may_take_the_place_of_v(L, bs, listed):
+    q, k, v = _qkv(L, 16, 16, seed=L)
+    lists = _lists(16, L, bs, 0.7) if listed else (None, None)
+    ref = block_sparse_attention(q, k, v, *lists, block_size=bs)
+    for shift in (0, 64 * 128):                      # v's own storage, and rows that meet it in part
+        buf = torch.zeros(shift + v.numel(), dtype=v.dtype, device=DEV)
+        buf[shift:] = v.transpose(1, 2).reshape(-1)
+        out = buf[:v.numel()].view(1, L, 16, 128)
+        got = block_sparse_attention(q, k, buf[shift:].view(1, L, 16, 128).transpose(1, 2), *lists, block_size=bs,
+                                     out=out)
+        assert torch.equal(got, ref)
