@@ -1182,7 +1182,7 @@ static bool out_meets_v(const fs_attn_args& a) {
 //          28 / 4 (57344): 213 / 209; 16384 (65536): 698 / 698, at D = 64 442 / 451.
 static bool v_direct(const fs_attn_args& a) {
   if (a.blk_cnt != nullptr && a.bs < 64) return false;   // union mode
-  if (a.v_sl >= (1 << 23)) return false;                 // 32-bit lane offsets
+  if (a.v_sl < 0 || a.v_sl >= (1 << 23)) return false;   // lane offsets are 32-bit, unsigned
   return (int64_t)(a.Hq / a.Hk) * a.Lk <= (a.blk_cnt != nullptr ? kDirectMaxKeys : kDirectMaxKeysDense);
 }
 

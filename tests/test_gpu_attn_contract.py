@@ -1,6 +1,6 @@
 """What a caller of the attention may rely on besides its result: the two halves
-of the call (prepare stages V, run reads what was staged), and an output that
-takes V's place."""
+of the call (prepare stages V, run reads what was staged), an output that takes
+V's place, and any stride of V."""
 from __future__ import annotations
 
 import pytest
@@ -64,3 +64,19 @@ def test_output_may_take_the_place_of_v(L, bs, listed):
         got = block_sparse_attention(q, k, buf[shift:].view(1, L, 16, 128).transpose(1, 2), *lists, block_size=bs,
                                      out=out)
         assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("step", [-1, 0])
+@pytest.mark.parametrize("listed", [False, True])
+def test_v_rows_in_descending_order_or_repeated(listed, step):
+    """Row strides of V that a C caller may give (torch has no negative ones)."""
+    L, H, D = 300, 2, 128
+    q, k, v = _qkv(L, H, H, seed=9)
+    lists = _lists(H, L, 64, 0.7) if listed else (None, None)
+    ref = block_sparse_attention(q, k, (v.flip(2) if step else v[:, :, :1].expand(-1, -1, L, -1)).contiguous(), *lists,
+                                 block_size=64)
+    call = AttentionCall(q, k, v, *lists, block_size=64)
+    if step:
+        call.args.v += 2 * (L - 1) * D               # each head's last row first
+    call.args.v_sl = step * D
+    assert torch.equal(call(), ref)
