@@ -42,6 +42,7 @@
 // and the same columns, which then hit that XCD's L2).
 // The dense path gives XCD x every 8th query-block row (last rows first) of
 // every head.
+#include <algorithm>
 #include <atomic>
 #include <climits>
 #include <type_traits>
@@ -1239,13 +1240,19 @@ static bool dense_by_64(const fs_attn_args& a, int Nq128) {
 // 32, at density 0.1 / 0.5 / 1 take 928 / 2328 / 2375 us by 128 and 747 / 2255 / 2633
 // by 64.  The lists are on the device, so the line is at the length alone.  At
 // D = 64 groups of 128 stay: 645 / 1592 / 1403 against 540 / 1651 / 1748.
-static int union_queries(const fs_attn_args& a) {
-  return a.D == 128 && a.Lk <= (a.bs == 32 ? kUnion64MaxKeys : kUnion64MaxKeys16) ? 64 : 128;
-}
-static int union_groups(const fs_attn_args& a) {
-  const int Nq = (a.Lq + a.bs - 1) / a.bs;
-  const int R = union_queries(a) / a.bs;
-  return (Nq + R - 1) / R;
+static int union64_max_keys(int bs) { return bs == 32 ? kUnion64MaxKeys : kUnion64MaxKeys16; }
+static int union_queries(const fs_attn_args& a) { return a.D == 128 && a.Lk <= union64_max_keys(a.bs) ? 64 : 128; }
+// Workspace of the union lists (u_cnt, then u_idx).  Groups of 64 write twice the
+// lists of groups of 128, so a call past their last length also gets the room of
+// the longest call in groups of 64 over its queries: a workspace sized for one
+// length serves every shorter one.
+static size_t union_bytes(const fs_attn_args& a) {
+  auto bytes = [&](int queries, int keys) {
+    const size_t R = queries / a.bs, Ng = ((size_t)(a.Lq + a.bs - 1) / a.bs + R - 1) / R, Nk = (keys + a.bs - 1) / a.bs;
+    return align256((size_t)a.Hq * Ng * sizeof(int32_t)) + (size_t)a.Hq * Ng * Nk * sizeof(uint32_t);
+  };
+  const size_t by128 = bytes(128, a.Lk);
+  return a.D == 128 ? std::max(by128, bytes(64, std::min(a.Lk, union64_max_keys(a.bs)))) : by128;
 }
 
 // order pass (block lists only) and the main kernel, reading V^T from the workspace
@@ -1351,10 +1358,7 @@ using namespace fs;
 extern "C" size_t fs_bsattn_work_bytes(const fs_attn_args* a) {
   if (!a || a->B <= 0 || a->Hq <= 0 || a->Hk <= 0 || a->Lq <= 0 || a->Lk <= 0 || a->D <= 0 || a->bs <= 0) return 0;
   size_t n = vt_bytes(*a) + order_bytes(*a);
-  if (union_mode(*a)) {
-    const size_t Ng = (size_t)union_groups(*a), Nk = (size_t)(a->Lk + a->bs - 1) / a->bs;
-    n += align256((size_t)a->Hq * Ng * sizeof(int32_t)) + (size_t)a->Hq * Ng * Nk * sizeof(uint32_t);
-  }
+  if (union_mode(*a)) n += union_bytes(*a);
   return n;
 }
 

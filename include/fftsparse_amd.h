@@ -351,7 +351,8 @@ FS_API int fs_flex(const fs_flex_args* a, void* stream);
  * work: fs_bsattn_work_bytes(a) bytes of device scratch (V may be staged there
  * transposed, and the work items' longest-first order and the counters from
  * which the attention kernel's workgroups take their work items are formed
- * there, before the attention kernel runs).  Calls that overlap on one
+ * there, before the attention kernel runs).  The size never falls with Lk, Lq, Hq
+ * or B, and a call without lists needs no more than one with them.  Calls that overlap on one
  * workspace race; the results do not depend on which workgroup takes
  * which item. */
 typedef struct {
