@@ -1204,22 +1204,31 @@ struct FlexLayout {
   size_t part, vert, slash, avgk, vmask, smask, info, attn, cover, p_hm, p_hc, c_hm, c_hc, ties, total;
 };
 
-// sparse: whether any head can take the block-level cover (tau > 0; the
-// square-root JS divergence is >= 0, or nan, so js < tau never holds otherwise)
 // Key columns per workgroup of the last-block passes: halved while the heads'
 // chunks leave workgroup slots empty (a chunk is a serial chain of 128-key
 // tiles), down to 512, where the second pass's extra tile per chunk costs a
 // fourth.  Both passes, 32 heads, 2048 against this: 8192 tokens 32-token blocks
 // 92 -> 47 us, 128-token blocks 262 -> 111; 32768 tokens 124 -> 121.
+constexpr int kFSlots = 1024;
 static int flex_chunk(int Hq, int L) {
   int c = kFChunk;
-  while (c > kFChunkMin && (int64_t)Hq * ((L + c - 1) / c) < 1024) c >>= 1;
+  while (c > kFChunkMin && (int64_t)Hq * ((L + c - 1) / c) < kFSlots) c >>= 1;
   return c;
 }
+// The most chunks of all heads that a call of up to Hq heads and L keys has: a
+// chunk below kFChunk is taken where chunks twice its size are fewer than
+// kFSlots, so they are fewer than twice that.  A workspace with room for these
+// serves every call with fewer heads or keys.
+static int64_t flex_max_chunks(int Hq, int L) {
+  const int64_t longest = (int64_t)Hq * ((L + kFChunk - 1) / kFChunk);
+  const int64_t shortest = (int64_t)Hq * ((L + kFChunkMin - 1) / kFChunkMin);
+  return std::max(longest, std::min<int64_t>(shortest, 2 * (kFSlots - 1)));
+}
 
+// sparse: whether any head can take the block-level cover (tau > 0; the
+// square-root JS divergence is >= 0, or nan, so js < tau never holds otherwise)
 static FlexLayout flex_work(int Hq, int Hk, int L, int bs, bool sparse) {
   const int nb = (L + bs - 1) / bs;
-  const int chunk = flex_chunk(Hq, L), nchunk = (L + chunk - 1) / chunk;
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t at = off;
@@ -1227,7 +1236,7 @@ static FlexLayout flex_work(int Hq, int Hk, int L, int bs, bool sparse) {
     return at;
   };
   FlexLayout w;
-  w.part = take((size_t)Hq * nchunk * bs * 2 * sizeof(float));
+  w.part = take((size_t)flex_max_chunks(Hq, L) * bs * 2 * sizeof(float));
   w.vert = take((size_t)Hq * L * sizeof(float));
   w.slash = take((size_t)Hq * L * sizeof(float));
   w.avgk = take((size_t)Hk * nb * kFD * sizeof(uint16_t));

@@ -315,7 +315,7 @@ FS_API int fs_xattn(const fs_xattn_args* a, void* stream);
  * and the per-token vertical / slash profiles [Hq][L] (fp32).
  * work: fs_flex_work_bytes(Hq, Hk, L, bs, tau) bytes, with the tau of the
  * call (tau <= 0, the reference's default, makes no head sparse and needs no
- * room for the block-level attention and covers).  bf16/f16, D = 128,
+ * room for the block-level attention and covers); the size never falls with L or Hq.  bf16/f16, D = 128,
  * bs 16, 32, 64 or 128, L > bs, N <= 8192. */
 typedef struct {
   const void* q; int64_t q_sh, q_sl;

@@ -35,3 +35,16 @@ def test_attention_workspace_grows_with_the_length(bs, D, Hq, Hk):
     for Lq in (1, 1000, 40000):
         n = [attn_bytes(L, bs, D, Hq, Hk, Lq=Lq) for L in LENGTHS]
         assert n == sorted(n)
+
+
+@pytest.mark.parametrize("bs", [16, 128])
+@pytest.mark.parametrize("tau", [0.0, 0.1])
+def test_flexprefill_workspace_grows_with_length_and_heads(bs, tau):
+    lib = _lib.load()
+    lengths = [L for L in LENGTHS if bs < L <= 8192 * bs] + list(range(60000, 70000, 509))
+    for Hq in (1, 4, 28, 32, 70, 512, 1024):
+        n = [lib.fs_flex_work_bytes(Hq, 1, L, bs, tau) for L in sorted(lengths)]
+        assert n == sorted(n)
+    for L in (300, 4100, 33000, 65537):
+        n = [lib.fs_flex_work_bytes(Hq, 1, L, bs, tau) for Hq in range(1, 1100, 3)]
+        assert n == sorted(n)
