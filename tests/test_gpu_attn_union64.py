@@ -56,3 +56,26 @@ def test_union_groups(L, bs, D, density, dtype):
     assert (got - ref).abs().max().item() <= 2 * eps * v.float().abs().max().item()
     empty = ~mask.any(-1)[:, rows // bs]
     assert (got[empty] == 0).all()
+
+
+@pytest.mark.parametrize("bs,D", [(32, 128), (16, 128), (32, 64), (16, 64)])
+def test_rows_that_begin_late_or_far_below_zero(bs, D):
+    """Rows whose first listed block comes after others' of the group (their first tiles hold no
+    key of theirs), with scores of -800 to -2300: from a start above them they would all be 0."""
+    L, H = 600, 2
+    n = -(-L // bs)
+    q = torch.full((1, H, L, D), 10.0, dtype=torch.bfloat16, device="cuda")
+    k = (-10.0 * (2.0 - torch.arange(L, device="cuda") / L))[None, None, :, None].expand(1, 1, L, D).bfloat16()
+    v = torch.randn(1, 1, L, D, generator=torch.Generator().manual_seed(bs)).bfloat16().cuda()
+    r, c = torch.meshgrid(torch.arange(n), torch.arange(n), indexing="ij")
+    mask = ((c >= r - r % 3) & (c <= r)).repeat(H, 1, 1)      # rows of a group begin 0, 1 or 2 blocks back
+    mask[1] &= (c == r)                                       # and the second head's at their own block
+    mask[:, 1::7] = False
+    cnt, bits = (t.cuda() for t in bits_from_mask(mask))
+    out = fftsparse_amd.block_sparse_attention(q, k.contiguous(), v, cnt, bits, block_size=bs)
+    j = torch.arange(L)
+    keep = mask[:, j // bs][:, :, j // bs] & (j[None] <= j[:, None])[None]
+    s = (q[0].double().cpu() @ k[0].double().cpu().expand(H, -1, -1).transpose(1, 2)) / D ** 0.5
+    p = torch.nan_to_num(torch.softmax(s.masked_fill(~keep, float("-inf")), -1))
+    ref = p @ v[0].double().cpu().expand(H, -1, -1)
+    assert (out.view(L, H, D).transpose(0, 1).double().cpu() - ref).abs().max() <= 2.0 ** -8 * v.abs().max().item()
