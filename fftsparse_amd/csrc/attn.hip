@@ -221,6 +221,7 @@ struct AttnKArgs {
   // last pool_units are taken by whichever XCD asks first
   int32_t* ctr;
   int static_units, pool_units;
+  float redo;                   // no row max: the row sum above which a tile is redone (redo_sum)
   int v_sl;                     // VD only: V's strides
   int64_t v_sb, v_sh;
 };
@@ -609,7 +610,7 @@ void bsattn_kernel(AttnKArgs a) {
   constexpr float kSlack = 8.0f;
   // Split tiles (block 64, two key groups of 16 MFMAs per wave) take their
   // exponentials against the running max with no row max: a tile whose row
-  // sum exceeds 2^64 (or is inf / nan, as on a row's first tile) is redone
+  // sum exceeds redo_sum (or is inf / nan, as on a row's first tile) is redone
   // with the raised max.  Against the row max: C3a -4.6%; at block 128 (32
   // MFMAs per wave) the row max is kept, the other form measured 3.5% slower.
   // At D = 64 a score costs the same softmax work beside half the MFMAs, the
@@ -852,7 +853,7 @@ void bsattn_kernel(AttnKArgs a) {
         if (__builtin_amdgcn_ballot_w64(al != 1.0f) != 0) scale_o(al);   // O holds P V up to t-1 now
       } else {
         float tot = r0 + r1;
-        const bool bad = !(tot <= 0x1p64f);            // p above 2^64 somewhere, inf or nan
+        const bool bad = !(tot <= a.redo);             // too large, inf or nan
         if (__builtin_amdgcn_ballot_w64(bad) != 0) {   // rare: the row's max, raised running max, exps again
           // the first pass's P stays defined before the branch (else its packing sinks out of the MFMA block)
 #pragma unroll
@@ -1223,6 +1224,12 @@ static int32_t* ticket_counters(const fs_attn_args& a) {
   return reinterpret_cast<int32_t*>(static_cast<char*>(a.work) + vt_bytes(a) +
                                     align256((size_t)a.Hq * Nq * sizeof(int32_t)));
 }
+// Row sum above which a tile whose exponentials were taken with no row max is
+// redone, i.e. how large P grows before the running max is raised.  O is a sum of
+// P V in fp32: 2^8 (the raise's slack with a row max) lets V reach what it may
+// reach there, 2^64 is the most that takes P to no infinity by itself.  f16 has
+// P <= 2^16 either way (past it P is inf) and V <= 2^16.
+static float redo_sum(const fs_attn_args& a) { return a.bs == 64 || a.dtype == FS_DTYPE_F16 ? 0x1p64f : 0x1p8f; }
 static bool union_mode(const fs_attn_args& a) { return a.blk_cnt != nullptr && a.bs < 64; }
 // Dense calls of few workgroups take 64 queries each instead of 128, so that
 // twice as many are in flight and a tile's keys are shared by two waves (the last
@@ -1310,6 +1317,7 @@ static int launch_run(const fs_attn_args& a, int Nq, int Nk, hipStream_t s, int 
   k.ctr = ctr;
   k.static_units = static_units;
   k.pool_units = pool_units;
+  k.redo = redo_sum(a);
   bsattn_kernel<BS, TK, T, BS, D, VD><<<grid, AttnCfg<BS, TK, D>::NT, 0, s>>>(k);
   return fs_host::launch_status("fs_bsattn");
 }
@@ -1354,6 +1362,7 @@ static int launch_run_union(const fs_attn_args& a, hipStream_t s) {
   k.scale = a.softmax_scale;
   k.ctr = ctr;
   k.gqa_interleave = a.gqa_interleave ? 1 : 0;
+  k.redo = redo_sum(a);
   const unsigned grid = deal_units(total, run, k.static_units, k.pool_units);
   bsattn_kernel<Q, 64, T, LB, D><<<grid, AttnCfg<Q, 64, D>::NT, 0, s>>>(k);
   return fs_host::launch_status("fs_bsattn");

@@ -1,7 +1,9 @@
 """What a caller of the attention may rely on besides its result: the two halves
 of the call (prepare stages V, run reads what was staged), an output that takes
-V's place, and any stride of V."""
+V's place, any stride of V, and large values."""
 from __future__ import annotations
+
+import math
 
 import pytest
 import torch
@@ -80,3 +82,25 @@ def test_v_rows_in_descending_order_or_repeated(listed, step):
         call.args.v += 2 * (L - 1) * D               # each head's last row first
     call.args.v_sl = step * D
     assert torch.equal(call(), ref)
+
+
+@pytest.mark.parametrize("D,bs,listed", [(64, 128, False), (64, 128, True), (64, 32, True), (64, 16, True),
+                                         (128, 128, False), (128, 32, True), (128, 16, True), (128, 128, True)])
+def test_large_values_under_rising_scores(D, bs, listed):
+    """Scores that rise along the keys by a factor of 2^55 in weight, values near 2^100: the output is
+    a mean of values, and the sums behind it stay finite too."""
+    L, H = 1000, 2
+    u = torch.nn.functional.normalize(torch.randn(D, generator=torch.Generator().manual_seed(D)), dim=0)
+    rise = torch.arange(L) / L * 55.0 * math.log(2.0) * D ** 0.5 / 8.0
+    q = (8.0 * u).expand(1, H, L, D).bfloat16().contiguous()
+    k = (rise[:, None] * u).expand(1, H, L, D).bfloat16().contiguous()
+    v = torch.randn(1, H, L, D, generator=torch.Generator().manual_seed(1)).bfloat16() * 2.0 ** 100
+    n = -(-L // bs)
+    lists = bits_from_mask(torch.ones(H, n, n, dtype=torch.bool)) if listed else (None, None)
+    out = block_sparse_attention(q.to(DEV), k.to(DEV), v.to(DEV), *(x.to(DEV) if listed else x for x in lists),
+                                 block_size=bs).double().cpu()
+    s = (q.double() @ k.double().transpose(-1, -2)) * D ** -0.5
+    s.masked_fill_(torch.ones(L, L, dtype=torch.bool).triu(1), float("-inf"))
+    ref = (torch.softmax(s, -1) @ (v.double() * 2.0 ** -100)).transpose(1, 2)
+    assert out.isfinite().all()
+    assert (out * 2.0 ** -100 - ref).abs().max() < 2e-2
