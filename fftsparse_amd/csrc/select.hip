@@ -447,17 +447,17 @@ __device__ void diffuse_rows(const fs_select_args& a, int h, int r0, int panel_r
 // gridDim.x, ..  (One workgroup per panel_rows rows of every head instead, the
 // stripe heads' spare ones returning: 21.6 against 10.1 us on 32 stripe heads of
 // 1024 blocks, the 64 KiB workgroups going through four rounds.)
-// Dynamic LDS: WordRowsLds (word-parallel rows), the head's flag bytes [N]
-// (other stripe rows), or the panel [panel_rows][N rounded up to 64] of keys.
+// Dynamic LDS (all there is, so that the panel's 64 KiB are a whole default
+// launch): the decisions, then WordRowsLds (word-parallel rows), the head's flag
+// bytes [N] (other stripe rows), or the panel [panel_rows][N rounded up to 64] of keys.
 template <typename T>
 __global__ __launch_bounds__(kSelThreads) __attribute__((amdgpu_waves_per_eu(4))) void select_kernel(
     fs_select_args a, int stripe_rows, int panel_rows, float inv_sqrt_d) {
   extern __shared__ __attribute__((aligned(16))) unsigned char sel_lds[];
-  __shared__ uint8_t is_diffuse[kHeadGroup];
-  const int N = a.N, Nk = a.Nk, D = a.D;
+  uint8_t* is_diffuse = sel_lds;                   // [kHeadGroup], before the first item
+  const int N = a.N;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: what follows from it branches on scalars
-  const int NW = (Nk + 63) >> 6;                   // 64-block words per row
   const int h0 = blockIdx.y * kHeadGroup, nh = min(kHeadGroup, a.Hq - h0);
 
   // ---- stripe / diffuse decisions (:359-363): wave w takes heads w, w + 8, .., four at a time
@@ -492,6 +492,7 @@ __global__ __launch_bounds__(kSelThreads) __attribute__((amdgpu_waves_per_eu(4))
     }
     __syncthreads();
     dmask = __ballot(lane < nh && is_diffuse[lane] != 0);
+    __syncthreads();                               // read before the items overwrite it
   }
   const uint64_t hmask = nh == 64 ? ~0ull : (1ull << nh) - 1;
   const int nd = __popcll(dmask), ns = nh - nd;
