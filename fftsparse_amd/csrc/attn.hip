@@ -984,7 +984,7 @@ constexpr int kTicketCounters = 9;               // 8 XCD shares + the shared po
 constexpr int kPoolPercent = 10;                 // share of the work units (the shortest) in the shared pool
 constexpr int kOrderMaxBins = 8192;
 constexpr int64_t kDirectMaxKeys = 49152;        // see v_direct
-constexpr int64_t kDirectMaxKeysDense = 24576;
+constexpr int64_t kDirectMaxKeysDense = 20480;
 constexpr int kUnion64MaxKeys = 40960;           // see union_queries
 constexpr int kUnion64MaxKeys16 = 32768;
 constexpr int kOrderKeysPerThread = 8;           // keys kept in registers between the two passes
@@ -1182,14 +1182,17 @@ static bool out_meets_v(const fs_attn_args& a) {
 }
 
 // fs_bsattn reads V as it is (no V^T pre-pass) where V is used few times: the
-// pre-pass moves V twice and is a launch (6 us at 1000 tokens, 26 us at 8192 with 32 KV
-// heads), the direct loop takes 1-3% longer, so the line is at a count of query
-// heads per KV head x keys.  Whole calls, V^T against direct, bf16, D = 128:
-//   dense  1000 tokens, 32 / 8 heads (4000): 29.5 / 23.6 us; 4096 (16384): 164 / 158;
-//          8192 (32768): 552 / 554; 16384 (65536): 2054 / 2067;
-//   lists  (density 0.3) 4096 (16384): 111 / 106 us; 8192 (32768): 229 / 224;
-//          32768 with 32 / 32 heads (32768): 2557 / 2513; block 64, 8192 with
-//          28 / 4 (57344): 213 / 209; 16384 (65536): 698 / 698, at D = 64 442 / 451.
+// pre-pass moves V twice and is a launch (6 us at 1000 tokens, 26 us at 8192 with
+// 32 KV heads), the direct loop takes 1-3% longer, so the line is at a count of
+// query heads per KV head x keys.  V^T against direct, 32 / 8 heads, bf16, D = 128
+// (D = 64):
+//   dense  1000 tokens (4000): 25.3 / 19.8 us (16.8 / 14.1); 2048 (8192): 55.1 / 50.4
+//          (37.1 / 33.4); 4096 (16384): 161.6 / 155.9 (98.2 / 93.3); 6000 (24000):
+//          311 / 313 (189 / 182), block 64 330 / 337 (208 / 212); 8192: 552 / 554;
+//   lists  (density 0.3) 4096 (16384): 94.6 / 89.6 us (65.6 / 60.8); 12000 (48000):
+//          470 / 471 (276 / 271), block 64 665 / 651 (356 / 361); 32768 with 32 / 32
+//          heads (32768): 3071 / 3079 (1739 / 1681); block 64, 7000 with 28 / 4
+//          (49000): 197 / 189 (137 / 136); 16384 (65536): 698 / 698 (442 / 451).
 static bool v_direct(const fs_attn_args& a) {
   if (a.blk_cnt != nullptr && a.bs < 64) return false;   // union mode
   if (a.v_sl < 0 || a.v_sl >= (1 << 23)) return false;   // lane offsets are 32-bit, unsigned
