@@ -561,10 +561,12 @@ extern "C" int fs_select(const fs_select_args* a, void* stream) {
   hipStream_t s = (hipStream_t)stream;
   const int dt = a->dyn_mode == 1 ? a->dtype : FS_DTYPE_F32;
   int rc = 0;
+  fs_select_args k = *a;
+  k.local_window = std::min(a->local_window, std::max(a->N, a->Nk));   // wider ones reach no further, and i + window overflows
   switch (dt) {
-    case FS_DTYPE_F32: rc = launch_select<float>(*a, grid, smem, stripe_rows, panel_rows, inv_sqrt_d, s); break;
-    case FS_DTYPE_BF16: rc = launch_select<bf16_t>(*a, grid, smem, stripe_rows, panel_rows, inv_sqrt_d, s); break;
-    case FS_DTYPE_F16: rc = launch_select<f16_t>(*a, grid, smem, stripe_rows, panel_rows, inv_sqrt_d, s); break;
+    case FS_DTYPE_F32: rc = launch_select<float>(k, grid, smem, stripe_rows, panel_rows, inv_sqrt_d, s); break;
+    case FS_DTYPE_BF16: rc = launch_select<bf16_t>(k, grid, smem, stripe_rows, panel_rows, inv_sqrt_d, s); break;
+    case FS_DTYPE_F16: rc = launch_select<f16_t>(k, grid, smem, stripe_rows, panel_rows, inv_sqrt_d, s); break;
     default: fs_host::set_error("fs_select: dtype %d unsupported", a->dtype); return FS_ERR_UNSUPPORTED;
   }
   if (rc) return rc;

@@ -95,3 +95,22 @@ def test_ties_at_the_threshold_go_to_the_lower_block():
         want = max(1, math.trunc(float(torch.tensor(float(i + 1)) * torch.tensor(0.3))))
         order = sorted(range(i + 1), key=lambda j: (j != 5, j))[:want]
         assert sorted(order) == torch.nonzero(m[i]).flatten().tolist()
+
+
+@pytest.mark.parametrize("diffuse", [True, False])
+@pytest.mark.parametrize("window", [2**31 - 1, 2**31 - 150, 199])
+def test_window_wider_than_the_sequence(diffuse, window):
+    """A local window that no sequence is long for selects every block up to the diagonal."""
+    N = 200
+    q_b = torch.randn(1, N, 64, generator=torch.Generator().manual_seed(2)).bfloat16().to(DEV)
+    cnt = torch.empty(1, N, dtype=torch.int32, device=DEV)
+    bits = torch.empty(1, N, (N + 63) // 64, dtype=torch.int64, device=DEV)
+    keep = torch.zeros(1, N, dtype=torch.uint8, device=DEV)
+    var = torch.zeros(1, 1, device=DEV)
+    _lib.call("fs_select", SelectArgs(
+        q_b=q_b.data_ptr(), k_b=q_b.data_ptr(), dtype=_lib.FS_DTYPE[torch.bfloat16], Hq=1, Hk=1, N=N, Nk=N, D=64,
+        mask_causal=1, keep_sink=0, keep_recent=0, local_window=window, remote_start=1, dyn_mode=1,
+        stripe_all_diffuse=int(diffuse), diag_var=var.data_ptr(), n_samples=1, stripe_threshold=1.0,
+        keep_tau=keep.data_ptr(), qk_topk_ratio=0.1, col_mode=0, blk_cnt=cnt.data_ptr(), blk_bits=bits.data_ptr()),
+        DEV)
+    assert cnt[0].cpu().tolist() == list(range(1, N + 1))
