@@ -1049,6 +1049,10 @@ __global__ __launch_bounds__(kFThreads) void flex_cover_rows_kernel(FlexCoverK a
       }
       l_run = l_run * expf(m_run - mx) + se;
       m_run = mx;
+    } else {
+      // no score above -inf yet: a nan among them still makes the row's sum nan
+#pragma unroll
+      for (int r = 0; r < 16; ++r) l_run = seen(t, r) && isnan(x[r]) ? x[r] : l_run;
     }
   });
   // the row's lanes: l32 and l32 + 32 of the four waves, merged in that order by each of them
@@ -1057,7 +1061,8 @@ __global__ __launch_bounds__(kFThreads) void flex_cover_rows_kernel(FlexCoverK a
   __syncthreads();
   float m = -INFINITY, se = 0.f;
   for (int e = l32; e < kFThreads; e += 32) m = fmaxf(m, red[e][0]);
-  for (int e = l32; e < kFThreads; e += 32) se += red[e][0] > -INFINITY ? red[e][1] * expf(red[e][0] - m) : 0.f;
+  // (a lane without a score above -inf: 0, or nan)
+  for (int e = l32; e < kFThreads; e += 32) se += red[e][0] > -INFINITY ? red[e][1] * expf(red[e][0] - m) : red[e][1];
   float* out = a.attn + ((int64_t)h * nb + row) * nb;
   tiles([&](int t, const float* x) {
     float p[16];

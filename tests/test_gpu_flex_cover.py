@@ -38,3 +38,24 @@ def test_cover_and_profiles_against_oracle(L, bs, Hq, Hk, dtype, tau):
     same = (got == ref.mask)[:, tri].float().mean().item()
     print(f"L={L} bs={bs} Hq={Hq}: equal {same:.6f} of {Hq * int(tri.sum())} decisions", flush=True)
     assert same >= 0.999
+
+
+@pytest.mark.parametrize("dims", [(0, 1), (0, 8), (0, 64)])
+@pytest.mark.parametrize("row,key", [(9, 4), (4, 4), (9, 9)])
+def test_score_past_the_float_range_spoils_its_whole_row(dims, row, key):
+    """A block score that leaves the float range (two dims of a query block and of a key block whose
+    products cancel) makes every probability of its row nan: the cover takes none of it, wherever in
+    the row the score lies, and the other rows as ever."""
+    n, bs, H = 12, 16, 1
+    q, k, _ = make_qkv(n * bs, H, H, dtype=torch.bfloat16, seed=bs)
+    qt, kt = q.transpose(1, 2).contiguous(), k.transpose(1, 2).contiguous()
+    qt[..., list(dims)] = 0.0
+    kt[..., list(dims)] = 0.0
+    qt[:, row * bs:(row + 1) * bs, :, list(dims)] = 1e30
+    kt[:, key * bs:(key + 1) * bs, :, dims[0]] = 1e30
+    kt[:, key * bs:(key + 1) * bs, :, dims[1]] = -1e30
+    sel = flex_select(qt.to(DEV), kt.to(DEV), gamma=0.9, tau=10.0, block_size=bs)
+    assert int(sel.head_info[0, 2]) == 1
+    got = sel.dense_mask().cpu()[0]
+    assert torch.nonzero(got[row]).flatten().tolist() == [0, row]
+    assert got.sum() > 2 * n
