@@ -248,7 +248,11 @@ __device__ __forceinline__ uint4 lds16(const char* base, uint32_t off) {
 // lane's scores of a key block its row did not select are masked.  A tile of TK
 // keys holds TK / LB union entries, so every K / V^T tile copy serves BS queries
 // and a wave works at the rate it has with BS-token blocks.  At BS = 64 and
-// LB = 32 each wave's share of a tile is one list row and one entry.
+// LB = 32 each wave's share of a tile is one list row and one entry.  Lists, work
+// order and tickets are always given here: tested at run time, the forms without
+// them cost these instances up to 17 scalar and 9 vector registers spilled in the
+// loop (without: FlexPrefill's lists of 32768 tokens 5642 -> 5237 us, full masks of
+// 16384 2541 -> 2353).
 //
 // VD (V direct): no V^T pre-pass.  V tiles are copied as they are, [TK][D], and
 // each operand of P V is two transposing LDS reads (ds_read_b64_tr_b16) instead
@@ -282,13 +286,13 @@ void bsattn_kernel(AttnKArgs a) {
   const int x = wg & 7, slot = wg >> 3;
   const int g = a.Hq / a.Hk;
   int b, h, qb;
-  if (a.order != nullptr) {
+  if (UNION || a.order != nullptr) {
     // block lists: units of `run` consecutive query blocks of one head, in
     // decreasing tile count, dealt round-robin to the XCDs; a unit's query
     // blocks take consecutive slots of one XCD, so they run side by side and
     // share the K/V tiles of their (shifted) lag diagonals and columns in its L2
     int unit, j;
-    if (a.ctr != nullptr) {
+    if (UNION || a.ctr != nullptr) {
       // Dynamic assignment: the workgroup takes the next ticket of its XCD's
       // share (the share's units in order, `run` consecutive tickets per unit,
       // so a unit's query blocks still run side by side on one XCD); once the
@@ -371,7 +375,7 @@ void bsattn_kernel(AttnKArgs a) {
   // their completion is tracked by lgkmcnt, so reading the next word never
   // waits on the tile copies in flight (vmcnt).
   typedef const __attribute__((address_space(4))) uint64_t* cptr64;
-  const bool listed = a.blk_cnt != nullptr;
+  const bool listed = UNION || a.blk_cnt != nullptr;
   int64_t lbase = 0;
   int cnt;                                         // key tiles of this query block
   int nb_listed = 0;                               // union entries
@@ -1249,15 +1253,18 @@ static bool dense_by_64(const fs_attn_args& a, int Nq128) {
 // 0.95: the rows select 76% of a union over 128 queries and 88% of one over 64
 // at 32-token blocks, 42% and 58% at 16) and gives a short call twice the workgroups,
 // but a tile copy serves half as many queries, and past the last-level cache the
-// copies bound the loop.  Whole FlexPrefill calls (gamma 0.95), 128 against 64:
-//   block 32, 32 / 8 heads: 4100 tokens 376 / 358 us, 9001 796 / 734, 32768 8010 /
-//     7705 (tau 0: 6238 / 5366), 65536 29.65 / 30.39 ms, 98304 63.8 / 64.8;
-//     32 / 32 heads: 40000 11120 / 10775 us; 16 / 2: 16000 1068 / 1025;
-//   block 16: 9000 (tau 0) 672 / 618, 30000 7172 / 7077.
-// Lists that select nearly everything lose: random masks of 16384 tokens, block
-// 32, at density 0.1 / 0.5 / 1 take 928 / 2328 / 2375 us by 128 and 747 / 2255 / 2633
-// by 64.  The lists are on the device, so the line is at the length alone.  At
-// D = 64 groups of 128 stay: 645 / 1592 / 1403 against 540 / 1651 / 1748.
+// copies bound the loop.  Attention over lists, 128 against 64 queries, us:
+//   FlexPrefill (gamma 0.95), block 32, 32 / 8 heads: 4100 tokens 165 / 144, 9001 554 /
+//     496, 32768 6533 / 5237; 8 / 8: 40000 2804 / 2340; block 16: 9000 533 / 473,
+//     30000 (16 / 4) 2832 / 2158; 65536, block 32: 24.7 / 21.8 ms on Gaussian inputs with
+//     sinks and stripes, 29.7 / 30.4 (whole calls) on ones with topics per segment too;
+//   random masks of 16384, block 32: density 0.1 840 / 718, 0.3 1705 / 1476, 0.5 2073 /
+//     1988, 0.7 2225 / 2325, 1 2102 / 2353; 30000, block 16, density 1 3965 / 4232;
+//   the 1280 tokens up to the diagonal: 16384, block 32 436 / 493; 9000, block 16 271 / 321.
+// So lists whose neighbouring rows select the same lose 5-19%.  The lists are on the
+// device and the line is at the length alone.  At D = 64 groups of 128 stay (random
+// masks of 16384, block 32, density 0.1, 0.5, 1: 590 / 469, 1416 / 1376, 1252 / 1489; the
+// 1280 tokens up to the diagonal 278 / 349).
 static int union64_max_keys(int bs) { return bs == 32 ? kUnion64MaxKeys : kUnion64MaxKeys16; }
 static int union_queries(const fs_attn_args& a) { return a.D == 128 && a.Lk <= union64_max_keys(a.bs) ? 64 : 128; }
 // Workspace of the union lists (u_cnt, then u_idx).  Groups of 64 write twice the
