@@ -58,6 +58,33 @@ def test_union_groups(L, bs, D, density, dtype):
     assert (got[empty] == 0).all()
 
 
+@pytest.mark.parametrize("Lk,bs", [(41003, 32), (32790, 16)])
+@pytest.mark.parametrize("Lq,causal,density,dtype", [
+    (700, True, 0.3, torch.float16), (333, False, 0.05, torch.bfloat16), (130, False, 1.0, torch.float16),
+    (260, True, 1.0, torch.bfloat16),
+])
+def test_groups_of_128_at_head_dim_128(Lk, bs, Lq, causal, density, dtype):
+    """Past the lengths of groups of 64: fewer queries than keys, not causal, full lists, both types."""
+    print(f"[case] groups of 128 Lk={Lk} bs={bs} Lq={Lq} causal={causal} density={density} {dtype}", flush=True)
+    Hq, D = 2, 128
+    g = torch.Generator(device="cuda").manual_seed(Lq + bs)
+    q, k, v = (torch.randn(1, h, n, D, generator=g, device="cuda").to(dtype) for h, n in ((Hq, Lq), (1, Lk), (1, Lk)))
+    mask = torch.rand(Hq, -(-Lq // bs), -(-Lk // bs), generator=g, device="cuda") < density
+    mask[:, 1::5] = False
+    cnt, bits = bits_from_mask(mask)
+    out = fftsparse_amd.block_sparse_attention(q, k, v, cnt, bits, block_size=bs, is_causal=causal)
+    i, j = torch.arange(Lq, device="cuda"), torch.arange(Lk, device="cuda")
+    for h in range(Hq):
+        s = q[0, h].float() @ k[0, 0].float().T.contiguous() * D ** -0.5
+        keep = mask[h][i // bs][:, j // bs]
+        if causal:
+            keep &= j[None] <= i[:, None] + Lk - Lq
+        p = torch.nan_to_num(torch.softmax(s.masked_fill(~keep, float("-inf")), -1))
+        eps = 2.0 ** (-9 if dtype == torch.bfloat16 else -12)
+        assert (out[0, :, h].float() - p @ v[0, 0].float()).abs().max() <= 2 * eps * v.float().abs().max()
+        assert (out[0, ~keep.any(-1), h] == 0).all()
+
+
 @pytest.mark.parametrize("bs,D", [(32, 128), (16, 128), (32, 64), (16, 64)])
 def test_rows_that_begin_late_or_far_below_zero(bs, D):
     """Rows whose first listed block comes after others' of the group (their first tiles hold no
