@@ -1147,6 +1147,21 @@ __global__ __launch_bounds__(64) void union_kernel(const uint64_t* __restrict__ 
   if (lane == 0) u_cnt[(int64_t)h * Ng + grp] = total;
 }
 
+// CUs of the current device, 0 if unknown
+static int cu_count() {
+  // read once per device; host threads may race to fill an entry, so it is
+  // atomic (they store the same value)
+  static std::atomic<int> cus[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  int n = cus[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 0;
+    cus[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
 // Work units go KV group by KV group (one KV head's K and V^T then stay in
 // the last-level cache while its query heads run) when a group's workgroups
 // fill at least 4 rounds of the device's workgroup slots (two per CU);
@@ -1155,18 +1170,8 @@ __global__ __launch_bounds__(64) void union_kernel(const uint64_t* __restrict__ 
 // per group, attention 2.03 -> 1.90 ms; configs 2 and 3 have 7 to 14 and
 // keep the grouped order, 2.2% and 0.8% faster with it).
 static int kv_major(const fs_attn_args& a, int Nq) {
-  // CU count per device, read once; host threads may race to fill an entry,
-  // so it is atomic (they store the same value)
-  static std::atomic<int> cus[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 1;
-  int n = cus[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 1;
-    cus[dev].store(n, std::memory_order_relaxed);
-  }
   const int64_t per_group = (int64_t)(a.Hq / a.Hk) * Nq;   // workgroups of one KV group
-  return per_group >= 4 * 2 * (int64_t)n ? 1 : 0;
+  return per_group >= 4 * 2 * (int64_t)cu_count() ? 1 : 0;
 }
 
 // Whether the output's storage meets V's (the spans of the two views, so views
@@ -1240,13 +1245,16 @@ static float redo_sum(const fs_attn_args& a) { return a.bs == 64 || a.dtype == F
 static bool union_mode(const fs_attn_args& a) { return a.blk_cnt != nullptr && a.bs < 64; }
 // Dense calls of few workgroups take 64 queries each instead of 128, so that
 // twice as many are in flight and a tile's keys are shared by two waves (the last
-// query block's chain of tiles is what such a call waits for).  128 against 64,
-// V direct, 32 / 8 heads: 1000 tokens (256 workgroups) 23.6 / 19.1 us, 2 x 768
-// (384) 27.0 / 22.7, 2048 (512) 53.4 / 50.2, 4 x 512 (512) 24.3 / 27.6, 4 x 1200
-// (1280) 74.5 / 80.4.
+// query block's chain of tiles is what such a call waits for): up to one and a
+// half workgroups per CU, long ones up to the two that a CU holds.  128 against
+// 64, V direct, 32 / 8 heads on 256 CUs: 1000 tokens (256 workgroups) 23.6 / 19.1
+// us, 2 x 768 (384) 27.0 / 22.7, 2048 (512) 53.4 / 50.2, 4 x 512 (512) 24.3 / 27.6,
+// 4 x 1200 (1280) 74.5 / 80.4.  The two forms add a row's keys in another order
+// (two halves merged at the end, or none), so a sequence's output may differ in
+// the last bit between calls of few and of many heads or sequences.
 static bool dense_by_64(const fs_attn_args& a, int Nq128) {
-  const int64_t wg = (int64_t)a.B * a.Hq * Nq128;
-  return wg <= 384 || (wg <= 512 && a.Lk >= 960);
+  const int64_t wg = (int64_t)a.B * a.Hq * Nq128, cus = cu_count();
+  return 2 * wg <= 3 * cus || (wg <= 2 * cus && a.Lk >= 960);
 }
 // Queries of a workgroup in union mode.  A group of 64 has fewer entries that
 // some of its rows did not select (FlexPrefill's lists of 32768 tokens, gamma

@@ -343,7 +343,9 @@ FS_API int fs_flex(const fs_flex_args* a, void* stream);
  * (NW = FS_MASK_WORDS(Nk); bits past the causal limit are ignored); blk_cnt
  * [Hq][Nq] (the rows' bit counts) only orders the work, largest first.
  * blk_cnt == NULL selects every key block up to the
- * causal limit (dense causal attention).  Supported: dtype bf16/f16, D in {64, 128},
+ * causal limit (dense causal attention; calls of few workgroups, i.e. short
+ * sequences and few heads, take 64 queries a workgroup and add a row's keys in
+ * another order, so the last bits depend on the whole call's size).  Supported: dtype bf16/f16, D in {64, 128},
  * bs in {16, 32, 64, 128} (16 and 32: FlexPrefill's block sizes; their masks
  * are attended 64 or 128 queries at a time (64 at D = 128 up to 40960 keys,
  * 32768 at bs = 16) over the union of those rows' lists, up to 8192 key blocks).  All tensors are
