@@ -93,8 +93,8 @@ class BlockSelection:
 
 
 # largest block count of the selection kernels: 8192 on the 16-bit path (block
-# scores on MFMA; a diffuse head's 4-row score panel in LDS), 4096 on the fp32
-# path (LDS FFT length 8192)
+# scores on MFMA; a diffuse head's score panel of two rows in 64 KiB of LDS),
+# 4096 on the fp32 path (LDS FFT length 8192)
 MAX_SELECT_BLOCKS = 8192
 MAX_FFT_BLOCKS = 4096
 

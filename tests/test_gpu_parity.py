@@ -358,8 +358,8 @@ def test_attention_running_max_raises(growth):
     (3000, 4, 1, torch.bfloat16, 0.05, True),     # sparse rows: union entries selected by one row only
 ])
 def test_attention_short_blocks(bs, L, Hq, Hk, dtype, density, causal):
-    """16- and 32-token blocks (a workgroup of 128 queries walks the union of
-    its 128 / bs rows' lists, masking per row) under random block lists of odd
+    """16- and 32-token blocks (a workgroup of 64 queries walks the union of
+    its 64 / bs rows' lists, masking per row) under random block lists of odd
     and even lengths, against fp32 attention under the same mask; and the
     dense causal path at that block size."""
     _print_case("attention-short-blocks", bs=bs, L=L, Hq=Hq, Hk=Hk, dtype=dtype, density=density, causal=causal)
